@@ -77,6 +77,8 @@ struct SoaAtoms {
     template <class Real> static __device__ __forceinline__ V3<Real> force(const DevSys& S, int i) {
         return ld3<Real>(S.force, S.atomStride, i);
     }
+    // a force as the array holds it
+    template <class Real> static __device__ __forceinline__ V3<Real> held_force(V3<Real> f) { return f; }
     // FP64 position of a free atom (hi + lo in mixed precision)
     template <class Real> static __device__ __forceinline__ V3<double> pos(const DevSys& S, int i) {
         return load_pos<Real>(S, i);
@@ -107,6 +109,14 @@ struct AdoptedAtoms {
         const size_t st = (size_t)S.ommStride;
         const double u = 1.0 / kFixedPointScale;
         return {(Real)((double)f[0] * u), (Real)((double)f[st] * u), (Real)((double)f[2 * st] * u)};
+    }
+    // a force as the fixed-point array holds it (OpenMM's conversion:
+    // truncation of f * 2^32)
+    static __device__ __forceinline__ long long fixed_point(double f) { return (long long)(f * kFixedPointScale); }
+    template <class Real> static __device__ __forceinline__ V3<Real> held_force(V3<Real> f) {
+        const double u = 1.0 / kFixedPointScale;
+        return {(Real)((double)fixed_point((double)f.x) * u), (Real)((double)fixed_point((double)f.y) * u),
+                (Real)((double)fixed_point((double)f.z) * u)};
     }
     template <class Real> static __device__ __forceinline__ V3<double> pos(const DevSys& S, int i) {
         const int s = S.ommSlot[i];

@@ -239,14 +239,26 @@ struct StepGraphs {
 // RigidBodyIntegrator::step(steps) on a context or a batch (`o` provides the
 // launches, its stream, graphs and switches).  With fusion the steps'
 // interior boundaries run as one fused pass each: part1, forces,
-// (steps - 1) x [fused, forces], part2.  With `refine` the last step is
+// (steps - 1) x [fused, forces], part2; where every force on an atom depends
+// on that atom alone, all of them before the last forces run in launches of
+// kStepsPerLaunch boundaries.  With `refine` the last step is
 // bracketed by the refined-energy kernels.  Only the last force evaluation
 // takes the potential energy (a step asks for forces alone); the graphs hold
 // the other steps, and the last one is launched on its own.
 template <class O> void run_steps(O& o, int steps, bool refine) {
     if (steps <= 0) return;
     const int tail = refine ? 1 : 0;
-    if (o.useFusion && steps >= 2) {
+    if (o.useFusion && steps >= 2 && o.localSteps()) {
+        // the steps' interior boundaries stay in registers (launch_steps)
+        o.launchSteps(steps - 1 - tail);
+        o.launchForces(!tail);
+        if (tail) {
+            o.launchRefineBegin(false);
+            o.launchFused();
+            o.launchForces(true);
+        }
+        o.launchPart2();
+    } else if (o.useFusion && steps >= 2) {
         int interior = steps - 1 - tail;
         o.launchPart1();
         o.launchForces(interior == 0 && !tail);
@@ -389,6 +401,9 @@ void time_phases(hipStream_t stream, int steps, const std::vector<std::function<
     }
 }
 
+// boundaries of a launchSteps call that a tuner times
+constexpr int kTuneBoundaries = 16;
+
 template <class P1, class F, class P2>
 void time_steps(hipStream_t stream, int steps, P1 p1, F f, P2 p2, double* avgMs, double* totalMs) {
     time_phases(stream, steps, {p1, f, p2}, avgMs, totalMs);
@@ -427,7 +442,7 @@ static size_t context_arena_bytes(size_t na, int numBodies, int numFree, int num
 static size_t tile_bytes_bound(size_t na, int numBodies, int numFree, int numClasses) {
     size_t part = ((size_t)numFree + 63) / 64 + ((size_t)numBodies + 63) / 64 + numClasses + 1;
     size_t force = (na + 63) / 64 + 1;
-    return (2 * part + force) * sizeof(Tile);
+    return (3 * part + force) * sizeof(Tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -495,7 +510,8 @@ struct rbhip_context {
     Tile* dPartTiles = nullptr;
     Tile* dForceTiles = nullptr;
     Tile* dSetupTiles = nullptr;
-    int nPartTiles = 0, nForceTiles = 0, nSetupTiles = 0;
+    Tile* dStepTiles = nullptr;                  // part tiles of kStepsBlock threads, for launchSteps
+    int nPartTiles = 0, nForceTiles = 0, nSetupTiles = 0, nStepTiles = 0;
     // cluster tiles, 64 clusters each: KE slots after the part tiles, and a
     // copy whose slots follow the set-up tiles
     Tile* dClusterTiles = nullptr;
@@ -718,15 +734,17 @@ struct rbhip_context {
     struct TileCache {
         int block = -1, shapesVersion = -1;
         std::map<int, int> lanes;
-        std::vector<Tile> part, force;
+        std::vector<Tile> part, force, step;
     };
     TileCache tileCache;
     const TileCache& tilesFor(int blk) {
         if (tileCache.block != blk || tileCache.lanes != lanes || tileCache.shapesVersion != shapesVersion) {
             tileCache.part = partTiles(blk, lanes);
             tileCache.force = forceTiles(blk);
+            tileCache.step = blk == kStepsBlock ? tileCache.part : partTiles(kStepsBlock, lanes);
             validateTiles(tileCache.part, blk, maxKeSlots);
             validateTiles(tileCache.force, blk, maxPeSlots);
+            validateTiles(tileCache.step, kStepsBlock, maxKeSlots);
             tileCache.block = blk;
             tileCache.shapesVersion = shapesVersion;
             tileCache.lanes = lanes;
@@ -746,6 +764,8 @@ struct rbhip_context {
         std::vector<Tile> ft = forceTiles(block);
         std::map<int, int> ones;
         std::vector<Tile> st = partTiles(setupBlock(), ones);
+        std::vector<Tile> kt = partTiles(kStepsBlock, lanes);
+        validateTiles(kt, kStepsBlock, maxKeSlots);
         validateTiles(pt, block, maxKeSlots);
         validateTiles(ft, block, maxPeSlots);
         validateTiles(st, setupBlock(), maxKeSlots);
@@ -755,6 +775,7 @@ struct rbhip_context {
         dPartTiles = tileArena.allocT<Tile>(pt.size() + 1);
         dForceTiles = tileArena.allocT<Tile>(ft.size() + 1);
         dSetupTiles = tileArena.allocT<Tile>(st.size() + 1);
+        dStepTiles = block == kStepsBlock ? dPartTiles : tileArena.allocT<Tile>(kt.size() + 1);
         std::vector<Tile> ct = clusterTiles((int)pt.size()), cst = clusterTiles((int)st.size());
         dClusterTiles = tileArena.allocT<Tile>(ct.size() + 1);
         dClusterSetupTiles = tileArena.allocT<Tile>(cst.size() + 1);
@@ -769,7 +790,10 @@ struct rbhip_context {
             HIPCHK(hipMemcpyAsync(dForceTiles, ft.data(), ft.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         if (!st.empty())
             HIPCHK(hipMemcpyAsync(dSetupTiles, st.data(), st.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
+        if (!kt.empty() && dStepTiles != dPartTiles)
+            HIPCHK(hipMemcpyAsync(dStepTiles, kt.data(), kt.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
+        nStepTiles = (int)kt.size();
         nPartTiles = (int)pt.size();
         nForceTiles = (int)ft.size();
         nSetupTiles = (int)st.size();
@@ -836,6 +860,26 @@ struct rbhip_context {
         HIPCHK(launch_fused(precision, rotationMode, dSys, dPartTiles, nPartTiles, block, maxBlocks, stream, layout()));
         launchClusters(CLUSTER_FUSED);
         launchSites();
+    }
+    // whether launchSteps can carry the system through several steps at once:
+    // no atom's force depends on another atom, and a lane's atoms fit its LDS
+    bool localSteps() const {
+        return !h.bondStart && numSites == 0 && numClusters == 0 &&
+               steps_lds_bytes(precision, atomsPerLane()) <= kStepsLdsMax;
+    }
+    // the most body atoms one lane holds
+    int atomsPerLane() const {
+        int m = 0;
+        for (const Class& c : classes) {
+            auto it = lanes.find(c.N);
+            const int L = it == lanes.end() ? 1 : it->second;
+            m = std::max(m, (c.N + L - 1) / L);
+        }
+        return m;
+    }
+    void launchSteps(int boundaries) {
+        HIPCHK(launch_steps(precision, rotationMode, dSys, dStepTiles, nStepTiles, boundaries, atomsPerLane(), stream,
+                            layout()));
     }
     int partKeSlots() const { return nPartTiles + nClusterTiles; }
     void launchRefineBegin(bool folded) {
@@ -1092,7 +1136,8 @@ struct rbhip_batch {
     DevSys* dSystems = nullptr;
     Tile* dPartTiles = nullptr;
     Tile* dForceTiles = nullptr;
-    int nPart = 0, nForce = 0;
+    Tile* dStepTiles = nullptr;                  // as a context's, over the members
+    int nPart = 0, nForce = 0, nStep = 0;
     std::vector<int> memberPartTiles, memberForceTiles;
     std::vector<int> memberVersions;             // sysVersion of each member's DevSys copy
     int* dKeSlots = nullptr;
@@ -1104,12 +1149,12 @@ struct rbhip_batch {
     void rebuild() {
         graphs.reset();
         arena.release();
-        nPart = nForce = 0;
+        nPart = nForce = nStep = 0;
         memberPartTiles.assign(members.size(), 0);
         memberForceTiles.assign(members.size(), 0);
         if (members.empty()) return;
         std::vector<DevSys> sys;
-        std::vector<Tile> pt, ft;
+        std::vector<Tile> pt, ft, kt;
         memberVersions.assign(members.size(), 0);
         size_t np = 0, nf = 0;
         for (rbhip_context* c : members) {
@@ -1126,15 +1171,19 @@ struct rbhip_batch {
             const auto& tc = c->tilesFor(block);
             for (Tile t : tc.part) { t.sys = (int)m; pt.push_back(t); }
             for (Tile t : tc.force) { t.sys = (int)m; ft.push_back(t); }
+            if (block != kStepsBlock)
+                for (Tile t : tc.step) { t.sys = (int)m; kt.push_back(t); }
             memberPartTiles[m] = (int)tc.part.size();
             memberForceTiles[m] = (int)tc.force.size();
         }
         // one launch order over every member's tiles (each keeps its
         // member's slot)
         pt = rbhip_context::launchOrder(pt);
+        kt = rbhip_context::launchOrder(kt);
         dSystems = arena.allocT<DevSys>(sys.size());
         dPartTiles = arena.allocT<Tile>(pt.size() + 1);
         dForceTiles = arena.allocT<Tile>(ft.size() + 1);
+        dStepTiles = block == kStepsBlock ? dPartTiles : arena.allocT<Tile>(kt.size() + 1);
         dKeSlots = arena.allocT<int>(members.size());
         dRed = arena.allocT<double>(4 * members.size());
         HIPCHK(hipMemcpyAsync(dSystems, sys.data(), sys.size() * sizeof(DevSys), hipMemcpyHostToDevice, stream));
@@ -1142,7 +1191,10 @@ struct rbhip_batch {
             HIPCHK(hipMemcpyAsync(dPartTiles, pt.data(), pt.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         if (!ft.empty())
             HIPCHK(hipMemcpyAsync(dForceTiles, ft.data(), ft.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
+        if (!kt.empty())
+            HIPCHK(hipMemcpyAsync(dStepTiles, kt.data(), kt.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
+        nStep = block == kStepsBlock ? (int)pt.size() : (int)kt.size();
         nPart = (int)pt.size();
         nForce = (int)ft.size();
     }
@@ -1187,6 +1239,21 @@ struct rbhip_batch {
     }
     void launchFused() {
         HIPCHK(launch_fused(precision, rotationMode, dSystems, dPartTiles, nPart, block, maxBlocks, stream, 0));
+    }
+    // as for a context, for every member at the batch's workgroup size
+    int atomsPerLane() const {
+        int m = 0;
+        for (const rbhip_context* c : members) m = std::max(m, c->atomsPerLane());
+        return m;
+    }
+    bool localSteps() const {
+        for (const rbhip_context* c : members)
+            if (c->h.bondStart || c->numSites > 0 || c->numClusters > 0) return false;
+        return steps_lds_bytes(precision, atomsPerLane()) <= kStepsLdsMax;
+    }
+    void launchSteps(int boundaries) {
+        HIPCHK(launch_steps(precision, rotationMode, dSystems, dStepTiles, nStep, boundaries, atomsPerLane(), stream,
+                            0));
     }
     void launchRefineBegin(bool folded) {
         HIPCHK(launch_refine_begin(precision, rotationMode, dSystems, dPartTiles, nPart, folded ? 1 : 0, block,
@@ -2535,12 +2602,18 @@ int rbhip_autotune(rbhip_context* ctx, int reps) {
             C.restoreSnapshot(snap, C.stream);
             HIPCHK(hipStreamSynchronize(C.stream));
         };
-        // the time of one step as rbhip_execute runs it: fused pass + forces
-        // with fusion, part1 + forces + part2 without
+        // the time of what rbhip_execute launches: a few steps in registers
+        // and their last forces and part 2 where it can, the fused pass +
+        // forces of one step with fusion, part1 + forces + part2 without
         auto measure = [&]() -> double {
             double avg[3], total;
             double t;
-            if (C.useFusion) {
+            if (C.useFusion && C.localSteps()) {
+                C.launchSteps(kTuneBoundaries); C.launchForces(); C.launchPart2();
+                time_phases(C.stream, reps, {[&] { C.launchSteps(kTuneBoundaries); }, [&] { C.launchForces(true); },
+                                             [&] { C.launchPart2(); }}, avg, &total);
+                t = avg[0] + avg[1] + avg[2];
+            } else if (C.useFusion) {
                 C.launchPart1(); C.launchForces();
                 C.launchFused(); C.launchForces();
                 time_phases(C.stream, reps, {[&] { C.launchFused(); }, [&] { C.launchForces(false); }}, avg, &total);
@@ -2811,10 +2884,15 @@ int rbhip_batch_autotune(rbhip_batch* batch, int reps) {
             for (size_t m = 0; m < B.members.size(); m++) B.members[m]->restoreSnapshot(*snaps[m], B.stream);
             HIPCHK(hipStreamSynchronize(B.stream));
         };
-        // time of one step as rbhip_batch_execute runs it
+        // time of what rbhip_batch_execute launches, as in rbhip_autotune
         auto measure = [&]() -> double {
             double avg[3], total, t;
-            if (B.useFusion) {
+            if (B.useFusion && B.localSteps()) {
+                B.launchSteps(kTuneBoundaries); B.launchForces(); B.launchPart2();
+                time_phases(B.stream, reps, {[&] { B.launchSteps(kTuneBoundaries); }, [&] { B.launchForces(true); },
+                                             [&] { B.launchPart2(); }}, avg, &total);
+                t = avg[0] + avg[1] + avg[2];
+            } else if (B.useFusion) {
                 B.launchPart1(); B.launchForces();
                 B.launchFused(); B.launchForces();
                 time_phases(B.stream, reps, {[&] { B.launchFused(); }, [&] { B.launchForces(false); }}, avg, &total);

@@ -85,6 +85,31 @@ template <class T> __device__ __forceinline__ Rot<T> rotT(Q4<T> q) {
 template <class T> __device__ __forceinline__ V3<T> apply(const Rot<T>& R, V3<T> x) {
     return {dot(R.r0, x), dot(R.r1, x), dot(R.r2, x)};
 }
+// The same for the step kernels, with every fused operation written out: the
+// compiler's own choice of which product of a sum to fuse depends on the code
+// around it, and kernels that must give one trajectory bit for bit (part 1 and
+// part 2, the fused pass, the steps kept in registers) would round d's rotation
+// differently.  YFIRST: the y product is the one rounded, else the x product.
+template <class T> __device__ __forceinline__ Rot<T> step_rot(Q4<T> q) {
+    const T bb = q.b * q.b, ac = q.a * q.c, ad = q.a * q.d, cd = q.c * q.d;
+    const T s = fma(q.a, q.a, bb), t = fma(q.a, q.a, -bb);
+    Rot<T> R;
+    R.r0 = {fma(-q.d, q.d, fma(-q.c, q.c, s)), (T)2 * fma(q.b, q.c, -ad), (T)2 * fma(q.b, q.d, ac)};
+    R.r1 = {(T)2 * fma(q.b, q.c, ad), fma(-q.d, q.d, fma(q.c, q.c, t)), (T)2 * fma(-q.a, q.b, cd)};
+    R.r2 = {(T)2 * fma(q.b, q.d, -ac), (T)2 * fma(q.a, q.b, cd), fma(q.d, q.d, fma(-q.c, q.c, t))};
+    return R;
+}
+template <bool YFIRST, class T> __device__ __forceinline__ T step_dot(V3<T> u, V3<T> v) {
+    return YFIRST ? fma(u.z, v.z, fma(u.x, v.x, u.y * v.y)) : fma(u.z, v.z, fma(u.y, v.y, u.x * v.x));
+}
+template <bool YFIRST, class T> __device__ __forceinline__ V3<T> step_apply(const Rot<T>& R, V3<T> x) {
+    return {step_dot<YFIRST>(R.r0, x), step_dot<YFIRST>(R.r1, x), step_dot<YFIRST>(R.r2, x)};
+}
+// for an atom's position: SMALL (bodies of 2 to 4 atoms on one lane under
+// NO-SQUISH) rounds the x product of the first row
+template <bool SMALL, class T> __device__ __forceinline__ V3<T> place_apply(const Rot<T>& R, V3<T> x) {
+    return {step_dot<!SMALL>(R.r0, x), step_dot<true>(R.r1, x), step_dot<true>(R.r2, x)};
+}
 
 // ---------------------------------------------------------------------------
 // sin(phi) and cos(phi) - 1.  The rotation below updates q <- q + q (cos-1)

@@ -30,6 +30,18 @@ hipError_t launch_free_ke(int precision, const DevSys* systems, const Tile* tile
 // part2 of step n and part1 of step n+1 in one pass (no atom velocities, no KE)
 hipError_t launch_fused(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
                         int block, int maxBlocks, hipStream_t stream, int adopted);
+// part 1, then `boundaries` x [forces, fused pass], of systems whose force on
+// an atom depends on that atom alone (no bonds, sites or constraints), each
+// launch carrying its bodies and free atoms through up to kStepsPerLaunch
+// boundaries; the force array is left as it was.  The tiles are those of
+// kStepsBlock-thread workgroups.  atomsPerLane: the most body atoms one lane
+// holds; a launch needs steps_lds_bytes of LDS, at most kStepsLdsMax.
+constexpr int kStepsBlock = 64;
+constexpr int kStepsPerLaunch = 64;
+constexpr size_t kStepsLdsMax = 64 << 10;
+size_t steps_lds_bytes(int precision, int atomsPerLane);
+hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
+                        int boundaries, int atomsPerLane, hipStream_t stream, int adopted);
 // refined energies of the systems whose refBody is set: the start terms of
 // the next step (`folded` = the stored momenta carry its first half-kick,
 // i.e. part1 follows; 0 = a fused boundary follows), the end terms after

@@ -13,6 +13,8 @@
 //            same F and torque, so folding it here is the same arithmetic).
 //   k_fused  part2 of step n + part1 of step n+1 in one pass (interior steps
 //            of RigidBodyIntegrator::step(k)).
+//   k_steps  several steps of systems whose atoms' forces depend on no other
+//            atom: part 1, then [forces, k_fused] boundaries, in registers.
 //   k_forces the force-field slot: harmonic tethers and harmonic bonds.
 //
 // Body state per body: q (Real4), body-frame L and p_cm (3 Reals each), iI =
@@ -87,6 +89,14 @@ template <class Real> __device__ __forceinline__ Body<Real> load_body(const DevS
 // more than 6 atoms, several lanes each)
 constexpr int STRIDED_BATCH = 8;
 
+// A(q)^T d of atom u of a lane's batch.  (The first of a batch rounds its y
+// product and the others their x product, as the compiler fused them when
+// these loops were tuned; one rule for all kernels keeps their trajectories
+// equal bit for bit.)
+template <class T> __device__ __forceinline__ V3<T> strided_apply(const Rot<T>& R, V3<T> d, int u) {
+    return u % STRIDED_BATCH == 0 ? step_apply<true>(R, d) : step_apply<false>(R, d);
+}
+
 // F = sum f_j and tau = sum delta_j x f_j in FP64, delta_j = A(q)^T d_j
 // Where body k (first atom atom0, N atoms) reads its body-fixed coordinates
 // and inertia: its own, or, in a tile of bodies that share them, those of
@@ -113,7 +123,7 @@ __device__ __forceinline__ void body_sums(const DevSys& S, const Rot<Real>& R, i
         }
 #pragma unroll
         for (int j = 0; j < NC; j++) {
-            V3<double> dl = cvt<double>(apply(R, dj[j]));
+            V3<double> dl = cvt<double>(step_apply<true>(R, dj[j]));
             V3<double> f = cvt<double>(fj[j]);
             F = F + f;
             tau = tau + cross(dl, f);
@@ -136,7 +146,7 @@ __device__ __forceinline__ void body_sums(const DevSys& S, const Rot<Real>& R, i
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 if (j0 + u * lanes < N) {
-                    V3<double> dl = cvt<double>(apply(R, dj[u]));
+                    V3<double> dl = cvt<double>(strided_apply(R, dj[u], u));
                     V3<double> f = cvt<double>(fj[u]);
                     F = F + f;
                     tau = tau + cross(dl, f);
@@ -170,7 +180,7 @@ __device__ __forceinline__ void body_sums_any(const DevSys& S, const Rot<Real>& 
 
 // atom positions r_cm + A(q)^T d_j: fp32 in mixed precision (the force field's
 // view; the exact value is rebuilt from the body state on download)
-template <class Real, int NC, class IO>
+template <class Real, bool EXACT, int NC, class IO>
 __device__ __forceinline__ void body_positions(const DevSys& S, const Rot<Real>& R, V3<double> rc, int atom0,
                                                int dbase, int N, int sub, int lanes) {
     if constexpr (NC > 0) {
@@ -178,7 +188,9 @@ __device__ __forceinline__ void body_positions(const DevSys& S, const Rot<Real>&
 #pragma unroll
         for (int j = 0; j < NC; j++) dj[j] = ld3<Real>(S.d, S.dStride, dbase + j);
 #pragma unroll
-        for (int j = 0; j < NC; j++) IO::template set_body_pos<Real>(S, atom0 + j, rc + cvt<double>(apply(R, dj[j])));
+        for (int j = 0; j < NC; j++)
+            IO::template set_body_pos<Real>(S, atom0 + j,
+                                            rc + cvt<double>(place_apply<(!EXACT && NC <= 4)>(R, dj[j])));
     } else {
         // loads of a batch first, then its stores (one round trip per batch)
         constexpr int U = STRIDED_BATCH;
@@ -190,24 +202,25 @@ __device__ __forceinline__ void body_positions(const DevSys& S, const Rot<Real>&
 #pragma unroll
             for (int u = 0; u < U; u++)
                 if (j0 + u * lanes < N)
-                    IO::template set_body_pos<Real>(S, atom0 + j0 + u * lanes, rc + cvt<double>(apply(R, dj[u])));
+                    IO::template set_body_pos<Real>(S, atom0 + j0 + u * lanes,
+                                                    rc + cvt<double>(strided_apply(R, dj[u], u)));
         }
     }
 }
 
-template <class Real, class IO>
+template <class Real, bool EXACT, class IO>
 __device__ __forceinline__ void body_positions_any(const DevSys& S, const Rot<Real>& R, V3<double> rc, int atom0,
                                                    int dbase, int N, int sub, int lanes) {
     if (lanes == 1) {
         switch (N) {
-        case 2: body_positions<Real, 2, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
-        case 3: body_positions<Real, 3, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
-        case 4: body_positions<Real, 4, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
-        case 6: body_positions<Real, 6, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
-        default: body_positions<Real, 0, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
+        case 2: body_positions<Real, EXACT, 2, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
+        case 3: body_positions<Real, EXACT, 3, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
+        case 4: body_positions<Real, EXACT, 4, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
+        case 6: body_positions<Real, EXACT, 6, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
+        default: body_positions<Real, EXACT, 0, IO>(S, R, rc, atom0, dbase, N, 0, 1); break;
         }
     } else {
-        body_positions<Real, 0, IO>(S, R, rc, atom0, dbase, N, sub, lanes);
+        body_positions<Real, EXACT, 0, IO>(S, R, rc, atom0, dbase, N, sub, lanes);
     }
 }
 
@@ -235,9 +248,24 @@ __device__ __forceinline__ void body_velocities(const DevSys& S, const Rot<Real>
     }
 }
 
-// A(q) x from the rows of A(q)^T
-template <class Real> __device__ __forceinline__ V3<double> to_body(const Rot<Real>& R, V3<double> x) {
-    return cvt<double>(R.r0) * x.x + cvt<double>(R.r1) * x.y + cvt<double>(R.r2) * x.z;
+// A(q) x from the rows of A(q)^T, fused operations written out as in
+// step_apply: the y product rounded, or the x product for the bodies whose
+// NO-SQUISH fused pass keeps them in registers (one lane, 2 to 4 atoms)
+template <class Real> __device__ __forceinline__ V3<double> to_body(const Rot<Real>& R, V3<double> x, bool small) {
+    const V3<double> r0 = cvt<double>(R.r0), r1 = cvt<double>(R.r1), r2 = cvt<double>(R.r2);
+    if (small)
+        return {fma(r2.x, x.z, fma(r1.x, x.y, r0.x * x.x)), fma(r2.y, x.z, fma(r1.y, x.y, r0.y * x.x)),
+                fma(r2.z, x.z, fma(r1.z, x.y, r0.z * x.x))};
+    return {fma(r2.x, x.z, fma(r0.x, x.x, r1.x * x.y)), fma(r2.y, x.z, fma(r0.y, x.x, r1.y * x.y)),
+            fma(r2.z, x.z, fma(r0.z, x.x, r1.z * x.y))};
+}
+// p + F h, fused (in part 2 the product is used twice, which would otherwise
+// be rounded there and not in the fused pass)
+__device__ __forceinline__ V3<double> kicked(V3<double> p, V3<double> F, double h) {
+    return {fma(F.x, h, p.x), fma(F.y, h, p.y), fma(F.z, h, p.z)};
+}
+__device__ __forceinline__ bool small_body(const DevSys& S, int N, int lanes) {
+    return S.rotationMode != 0 && lanes == 1 && N <= 4;
 }
 
 // body-frame torque; a linear body (1/I2 = 0) has no moment about its axis
@@ -359,7 +387,7 @@ __device__ __forceinline__ void part1_bodies(const DevSys& S, const Tile& tile) 
         stp3<Real>(S.L, k, B.L);
         store_rcm<Real>(S, k, rc);
     }
-    body_positions_any<Real, IO>(S, rotT(B.q), rc, atom0, dbase, tile.N, sub, tile.lanes);
+    body_positions_any<Real, EXACT, IO>(S, step_rot(B.q), rc, atom0, dbase, tile.N, sub, tile.lanes);
 }
 
 // How a step kernel holds its system descriptor.  The exact-rotation kernels
@@ -415,14 +443,14 @@ __device__ __forceinline__ void part2_bodies(const DevSys& S, const Tile& tile, 
     const Shape sh = body_shape(S, tile, k, atom0, N);
     const int dbase = sh.row;
     Body<Real> B = load_body<Real>(S, k, sh.ks);
-    Rot<Real> R = rotT(B.q);
+    Rot<Real> R = step_rot(B.q);
     V3<double> F, tau;
     body_sums_any<Real, IO>(S, R, atom0, dbase, N, sub, tile.lanes, active, F, tau);
     if (!active) return;
     const double halfDt = 0.5 * S.dt;
-    V3<double> tb = axial_torque(to_body(R, tau), B.invI);
-    V3<double> p = cvt<double>(B.p) + F * halfDt;
-    V3<double> L = cvt<double>(B.L) + tb * halfDt;
+    V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
+    V3<double> p = kicked(cvt<double>(B.p), F, halfDt);
+    V3<double> L = kicked(cvt<double>(B.L), tb, halfDt);
     V3<double> w = hadamard(cvt<double>(B.invI), L);
     V3<double> vcm = p * (double)B.invM;
     V3<Real> ws = apply(R, cvt<Real>(w));
@@ -437,8 +465,8 @@ __device__ __forceinline__ void part2_bodies(const DevSys& S, const Tile& tile, 
         ke[0] = dot(p, vcm);
         ke[1] = dot(L, w);
         // first half-kick of the next step (same F and torque)
-        stp3<Real>(S.pcm, k, cvt<Real>(p + F * halfDt));
-        stp3<Real>(S.L, k, cvt<Real>(L + tb * halfDt));
+        stp3<Real>(S.pcm, k, cvt<Real>(kicked(p, F, halfDt)));
+        stp3<Real>(S.L, k, cvt<Real>(kicked(L, tb, halfDt)));
     }
 }
 
@@ -485,13 +513,13 @@ __device__ __forceinline__ void fused_free(const DevSys& S, const Tile& tile) {
 // part2 of step n and the first half-kick of step n+1 on the body momenta
 template <class Real>
 __device__ __forceinline__ void fused_kicks(const DevSys& S, Body<Real>& B, const Rot<Real>& R, V3<double> F,
-                                            V3<double> tau) {
+                                            V3<double> tau, bool small) {
     const double halfDt = 0.5 * S.dt;
-    V3<double> tb = axial_torque(to_body(R, tau), B.invI);
-    V3<double> p = cvt<double>(B.p) + F * halfDt;
-    V3<double> L = cvt<double>(B.L) + tb * halfDt;
-    B.p = cvt<Real>(p + F * halfDt);
-    B.L = cvt<Real>(L + tb * halfDt);
+    V3<double> tb = axial_torque(to_body(R, tau, small), B.invI);
+    V3<double> p = kicked(cvt<double>(B.p), F, halfDt);
+    V3<double> L = kicked(cvt<double>(B.L), tb, halfDt);
+    B.p = cvt<Real>(kicked(p, F, halfDt));
+    B.L = cvt<Real>(kicked(L, tb, halfDt));
 }
 
 template <class Real> __device__ __forceinline__ void store_body(const DevSys& S, int k, const Body<Real>& B,
@@ -514,21 +542,22 @@ __device__ __forceinline__ void fused_body_regs(const DevSys& S, int k, int atom
         dj[j] = ld3<Real>(S.d, S.dStride, dbase + j);
         fj[j] = IO::template force<Real>(S, atom0 + j);
     }
-    Rot<Real> R = rotT(B.q);
+    Rot<Real> R = step_rot(B.q);
     V3<double> F = {0.0, 0.0, 0.0}, tau = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int j = 0; j < NC; j++) {
-        V3<double> dl = cvt<double>(apply(R, dj[j]));
+        V3<double> dl = cvt<double>(step_apply<true>(R, dj[j]));
         V3<double> f = cvt<double>(fj[j]);
         F = F + f;
         tau = tau + cross(dl, f);
     }
-    fused_kicks<Real>(S, B, R, F, tau);
+    fused_kicks<Real>(S, B, R, F, tau, true);
     drift_and_rotate<Real, EXACT>(S, B, rc);
     store_body<Real>(S, k, B, rc);
-    Rot<Real> R1 = rotT(B.q);
+    Rot<Real> R1 = step_rot(B.q);
 #pragma unroll
-    for (int j = 0; j < NC; j++) IO::template set_body_pos<Real>(S, atom0 + j, rc + cvt<double>(apply(R1, dj[j])));
+    for (int j = 0; j < NC; j++)
+        IO::template set_body_pos<Real>(S, atom0 + j, rc + cvt<double>(place_apply<!EXACT>(R1, dj[j])));
 }
 
 template <class Real, bool EXACT, class IO>
@@ -555,14 +584,14 @@ __device__ __forceinline__ void fused_bodies(const DevSys& S, const Tile& tile) 
     const int dbase = sh.row;
     Body<Real> B = load_body<Real>(S, k, sh.ks);
     V3<double> rc = load_rcm<Real>(S, k);
-    Rot<Real> R = rotT(B.q);
+    Rot<Real> R = step_rot(B.q);
     V3<double> F, tau;
     body_sums_any<Real, IO>(S, R, atom0, dbase, N, sub, tile.lanes, active, F, tau);
     if (!active) return;
-    fused_kicks<Real>(S, B, R, F, tau);
+    fused_kicks<Real>(S, B, R, F, tau, small_body(S, N, tile.lanes));
     drift_and_rotate<Real, EXACT>(S, B, rc);
     if (sub == 0) store_body<Real>(S, k, B, rc);
-    body_positions_any<Real, IO>(S, rotT(B.q), rc, atom0, dbase, N, sub, tile.lanes);
+    body_positions_any<Real, EXACT, IO>(S, step_rot(B.q), rc, atom0, dbase, N, sub, tile.lanes);
 }
 
 template <class Real, bool EXACT, class IO>
@@ -640,11 +669,11 @@ __device__ __forceinline__ void refine_begin_bodies(const DevSys& S, const Tile&
     const int atom0 = tile.atomFirst + (active ? b : 0) * tile.N;
     const Shape sh = body_shape(S, tile, k, atom0, tile.N);
     Body<Real> B = load_body<Real>(S, k, sh.ks);
-    Rot<Real> R = rotT(B.q);
+    Rot<Real> R = step_rot(B.q);
     V3<double> F, tau;
     body_sums_any<Real, IO>(S, R, atom0, sh.row, tile.N, sub, tile.lanes, active, F, tau);
     if (!active || sub != 0) return;
-    V3<double> tb = axial_torque(to_body(R, tau), B.invI);
+    V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
     V3<double> ar;
     V3<Real> Lback;
     Body<Real> B1 = B;
@@ -654,7 +683,7 @@ __device__ __forceinline__ void refine_begin_bodies(const DevSys& S, const Tile&
         Lback = cvt<Real>(cvt<double>(B.L) + tb * -S.dt);
     } else {
         // stored p = p(t-dt/2), L = L(t) - tau dt/2 (after the last rotation)
-        fused_kicks<Real>(S, B1, R, F, tau);
+        fused_kicks<Real>(S, B1, R, F, tau, small_body(S, tile.N, tile.lanes));
         ar = cvt<double>(B1.p) * 5.0 + cvt<double>(B.p) * -1.0;
         Lback = B.L;
     }
@@ -706,12 +735,12 @@ __device__ __forceinline__ void refine_end_bodies(const DevSys& S, const Tile& t
     // stored after part2: q(t+dt), p and L with the next half-kick folded in
     const Shape sh = body_shape(S, tile, k, atom0, tile.N);
     Body<Real> B = load_body<Real>(S, k, sh.ks);
-    Rot<Real> R = rotT(B.q);
+    Rot<Real> R = step_rot(B.q);
     V3<double> F, tau;
     body_sums_any<Real, IO>(S, R, atom0, sh.row, tile.N, sub, tile.lanes, active, F, tau);
     if (!active || sub != 0) return;
     const double halfDt = 0.5 * S.dt;
-    V3<double> tb = axial_torque(to_body(R, tau), B.invI);
+    V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
     V3<double> p1 = cvt<double>(B.p) + F * -halfDt;
     V3<double> L1 = cvt<double>(B.L) + tb * -halfDt;
     Q4<Real> r0 = ld4<Real>(S.refBody, 2 * k), r1 = ld4<Real>(S.refBody, 2 * k + 1);
@@ -769,11 +798,11 @@ __global__ __launch_bounds__(512) void k_refine_pe(const DevSys* __restrict__ sy
             const int atom0 = tile.atomFirst + (active ? b : 0) * tile.N;
             const Shape sh = body_shape(S, tile, k, atom0, tile.N);
             Body<Real> B = load_body<Real>(S, k, sh.ks);
-            Rot<Real> R = rotT(B.q);
+            Rot<Real> R = step_rot(B.q);
             V3<double> F, tau;
             body_sums_any<Real, IO>(S, R, atom0, sh.row, tile.N, sub, tile.lanes, active, F, tau);
             if (active && sub == 0) {
-                V3<double> tb = axial_torque(to_body(R, tau), B.invI);
+                V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
                 u[0] = dot(F, F) * (double)B.invM + dot(hadamard(tb, cvt<double>(B.invI)), tb);
             }
         }
@@ -1221,14 +1250,13 @@ template <class Real, class IO = SoaAtoms> __device__ __forceinline__ V3<double>
     return cvt<double>(hi) + cvt<double>(lo);
 }
 // a force into the library's array, or into the adopted fixed-point array
-// (OpenMM's conversion: truncation of f * 2^32)
 template <class Real, class IO> __device__ __forceinline__ void store_force(const DevSys& S, int i, V3<Real> f) {
     if constexpr (IO::adopted) {
         long long* o = S.ommForce + S.ommSlot[i];
         const size_t st = (size_t)S.ommStride;
-        o[0] = (long long)((double)f.x * kFixedPointScale);
-        o[st] = (long long)((double)f.y * kFixedPointScale);
-        o[2 * st] = (long long)((double)f.z * kFixedPointScale);
+        o[0] = IO::fixed_point((double)f.x);
+        o[st] = IO::fixed_point((double)f.y);
+        o[2 * st] = IO::fixed_point((double)f.z);
     } else {
         st3<Real>(S.force, S.atomStride, i, f);
     }
@@ -1342,6 +1370,13 @@ __global__ __launch_bounds__(256) void k_site_clear(const DevSys* __restrict__ s
 // the energy at its last evaluation alone.
 // ---------------------------------------------------------------------------
 
+// -k dx, rounded (never fused into the sum it goes to, so a force summed in
+// registers equals one that went through the force array)
+template <class Real> __device__ __forceinline__ V3<Real> tether_force(V3<Real> dx, Real k) {
+#pragma clang fp contract(off)
+    return {dx.x * (-k), dx.y * (-k), dx.z * (-k)};
+}
+
 template <class Real, class IO, bool ENERGY>
 __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ systems, const Tile* __restrict__ tiles,
                                                  int numTiles) {
@@ -1360,7 +1395,7 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
                 V3<Real> ph, pl;
                 field_pos_parts<Real, IO>(S, a, ph, pl);
                 V3<Real> dx = (ph - ld3<Real>(S.r0, S.atomStride, a)) + pl;
-                f = dx * (-k);
+                f = tether_force(dx, k);
                 if (ENERGY) {
                     V3<double> dd = cvt<double>(dx);
                     e[0] += 0.5 * (double)k * dot(dd, dd);
@@ -1384,6 +1419,188 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
             store_force<Real, IO>(S, a, f);
         }
         if (ENERGY) block_reduce_store<1>(e, S.pePart, tile.slot);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Steps of systems whose force on an atom depends on that atom alone (no
+// bonds, sites or constraints: the tether, or no force).  A body's interior
+// step boundaries then need nothing from other bodies, so one launch carries
+// each body (each free atom) through `boundaries` x [forces, fused pass] with
+// its state in registers and its atoms' coordinates and anchors in LDS:
+// positions, forces and body state go through memory once per launch instead
+// of once per step.  The arithmetic and every rounding to the state precision
+// are those of k_part1, k_forces and k_fused (the fused operations whose
+// choice the compiler makes by context are written out: step_rot, step_apply,
+// to_body, kicked), so results are the same bit for bit.
+// FIRST: a part 1 comes before the boundaries; LAST: the atom positions are
+// written at the end (a launch that continues another reads only the body
+// state).
+//
+// What bounds it: VALU issue (NO-SQUISH: 41 turns of 24 instructions in the
+// ~1300 of a body's step; FP64 latency with the exact rotation), no longer
+// HBM.  Per step, k_fused + k_forces -> k_steps: 1M waters, NO-SQUISH 10,
+// 58.2 -> 23.4 us; 20k waters 9.9 -> 2.8 us; the heterogeneous mix (200k
+// bodies, 500k free atoms, exact) 32.5 -> 8.6 us; 512 waters in FP64, exact,
+// 9.3 -> 3.2 us.  One wave per workgroup: tiles end apart, and the launch
+// fills the SIMDs evenly.  kStepsPerLaunch: 16, 64, 256 and 2048 boundaries
+// per launch ran the 1M waters at 24.0, 23.4, 23.8 and 23.8 us and the
+// heterogeneous mix at 9.2, 8.6, 8.6 and 8.7; 64 leaves other streams a slot
+// every few ms (a server's set-ups: 29 against 31 ms for a backlog with 2048).
+//
+// LDS: each lane keeps its own atoms' {d, r0, k}, 7 Reals per atom, at an odd
+// stride of Reals, so the lanes of a wave hit different banks; a lane reads
+// only what it wrote, so there is no barrier.  One copy of the rotation
+// serves every body size (the sizes differ in the sums only): with one per
+// size the exact kernel needed 256 + 14 registers and ran one wave per SIMD.
+// ---------------------------------------------------------------------------
+enum : int { STEPS_FIRST = 1, STEPS_LAST = 2 };
+
+// adds one tethered atom's force and torque to F and tau (a: its {d, r0, k})
+template <class Real, bool YFIRST, bool SMALL, class IO>
+__device__ __forceinline__ void add_tethered(const Real* a, bool uniform, Real k0, const Rot<Real>& R, V3<double> rc,
+                                             V3<double>& F, V3<double>& tau) {
+    const V3<Real> d = {a[0], a[1], a[2]};
+    V3<double> dl = cvt<double>(step_apply<YFIRST>(R, d));
+    V3<Real> x = cvt<Real>(rc + (SMALL ? cvt<double>(place_apply<true>(R, d)) : dl));
+    V3<double> f = cvt<double>(IO::held_force(tether_force(x - V3<Real>{a[3], a[4], a[5]}, uniform ? k0 : a[6])));
+    F = F + f;
+    tau = tau + cross(dl, f);
+}
+
+// F and tau of one body's (or one lane's share of its) atoms at st, in the
+// order and with the rounding of body_sums (N: the body's atoms if one lane
+// has them all)
+template <class Real, bool EXACT, class IO>
+__device__ __forceinline__ void tethered_sums(const Real* st, int N, int per, bool uniform, Real k0,
+                                              const Rot<Real>& R, V3<double> rc, V3<double>& F, V3<double>& tau) {
+    auto fixed = [&](auto NC) {
+#pragma unroll
+        for (int u = 0; u < NC; u++)
+            add_tethered<Real, true, (!EXACT && decltype(NC)::value <= 4), IO>(st + 7 * u, uniform, k0, R, rc, F, tau);
+    };
+    switch (N) {
+    case 2: fixed(std::integral_constant<int, 2>{}); break;
+    case 3: fixed(std::integral_constant<int, 3>{}); break;
+    case 4: fixed(std::integral_constant<int, 4>{}); break;
+    case 6: fixed(std::integral_constant<int, 6>{}); break;
+    default:
+        for (int u0 = 0; u0 < per; u0 += STRIDED_BATCH) {
+            add_tethered<Real, true, false, IO>(st + 7 * u0, uniform, k0, R, rc, F, tau);
+            const int end = per < u0 + STRIDED_BATCH ? per : u0 + STRIDED_BATCH;
+            for (int u = u0 + 1; u < end; u++)
+                add_tethered<Real, false, false, IO>(st + 7 * u, uniform, k0, R, rc, F, tau);
+        }
+    }
+}
+
+template <class Real, bool EXACT, class IO>
+__device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, int boundaries, int flags,
+                                             Real* stash) {
+    const int N = tile.N, lanes = tile.lanes;
+    const int b = threadIdx.x >> lane_shift(lanes);
+    const int sub = threadIdx.x & (lanes - 1);
+    if (b >= tile.count) return;
+    const int k = tile.first + b;
+    const int atom0 = tile.atomFirst + b * N;
+    const Shape sh = body_shape(S, tile, k, atom0, N);
+    const int perMax = (N + lanes - 1) / lanes;
+    const int per = (N - sub + lanes - 1) / lanes;
+    Real* st = stash + (size_t)threadIdx.x * ((7 * perMax) | 1);
+    const bool tethered = S.tetherScale != 0.0, uniform = S.tetherUniform != 0;
+    const Real k0 = (Real)S.tetherK0;
+    for (int u = 0; u < per; u++) {
+        const int j = sub + u * lanes;
+        V3<Real> d = ld3<Real>(S.d, S.dStride, sh.row + j);
+        V3<Real> r0 = ld3<Real>(S.r0, S.atomStride, atom0 + j);
+        Real* a = st + 7 * u;
+        a[0] = d.x; a[1] = d.y; a[2] = d.z;
+        a[3] = r0.x; a[4] = r0.y; a[5] = r0.z;
+        a[6] = uniform ? k0 : reinterpret_cast<const Real*>(S.tetherK)[atom0 + j];
+    }
+    Body<Real> B = load_body<Real>(S, k, sh.ks);
+    V3<double> rc = load_rcm<Real>(S, k);
+    const bool small = small_body(S, N, lanes);
+    const int first = (flags & STEPS_FIRST) ? -1 : 0;
+    for (int s = first; s < boundaries; s++) {
+        if (s >= 0) {
+            Rot<Real> R = step_rot(B.q);
+            V3<double> F = {0.0, 0.0, 0.0}, tau = {0.0, 0.0, 0.0};
+            if (tethered) tethered_sums<Real, EXACT, IO>(st, lanes == 1 ? N : 0, per, uniform, k0, R, rc, F, tau);
+            if (lanes > 1) {
+                F = {xor_sum(F.x, lanes), xor_sum(F.y, lanes), xor_sum(F.z, lanes)};
+                tau = {xor_sum(tau.x, lanes), xor_sum(tau.y, lanes), xor_sum(tau.z, lanes)};
+            }
+            fused_kicks<Real>(S, B, R, F, tau, small);
+        }
+        drift_and_rotate<Real, EXACT>(S, B, rc);
+    }
+    if (sub == 0) store_body<Real>(S, k, B, rc);
+    if (flags & STEPS_LAST) {
+        Rot<Real> R = step_rot(B.q);
+        const bool fixed = lanes == 1 && (N == 2 || N == 3 || N == 4 || N == 6);
+        for (int u = 0; u < per; u++) {
+            const V3<Real> d = {st[7 * u], st[7 * u + 1], st[7 * u + 2]};
+            const V3<Real> dl = !fixed ? strided_apply(R, d, u) : small ? place_apply<true>(R, d) : step_apply<true>(R, d);
+            IO::template set_body_pos<Real>(S, atom0 + sub + u * lanes, rc + cvt<double>(dl));
+        }
+    }
+}
+
+template <class Real, class IO>
+__device__ __forceinline__ void steps_free(const DevSys& S, const Tile& tile, int boundaries, int flags) {
+    const Real halfDt = (Real)(0.5 * S.dt);
+    const bool tethered = S.tetherScale != 0.0, uniform = S.tetherUniform != 0;
+    for (int i = threadIdx.x; i < tile.count; i += blockDim.x) {
+        const int a = tile.first + i;
+        V3<Real> v = IO::template vel<Real>(S, a);
+        const Real invm = reinterpret_cast<const Real*>(S.freeInvM)[a];
+        const V3<Real> r0 = ld3<Real>(S.r0, S.atomStride, a);
+        const Real k = uniform ? (Real)S.tetherK0 : reinterpret_cast<const Real*>(S.tetherK)[a];
+        V3<double> r = IO::template pos<Real>(S, a);
+        // the stored position: hi + lo in mixed precision
+        V3<Real> hi = cvt<Real>(r), lo = {(Real)0, (Real)0, (Real)0};
+        auto split = [&] {
+            hi = cvt<Real>(r);
+            if (sizeof(Real) == 4) {
+                lo = cvt<Real>(r - cvt<double>(hi));
+                r = cvt<double>(hi) + cvt<double>(lo);
+            }
+        };
+        split();
+        if (flags & STEPS_FIRST) {
+            V3<Real> f = IO::template force<Real>(S, a);
+            v = v + f * invm * halfDt;
+            r = r + cvt<double>(v) * S.dt;
+            split();
+        }
+        for (int s = 0; s < boundaries; s++) {
+            V3<Real> f = {(Real)0, (Real)0, (Real)0};
+            if (tethered) f = IO::held_force(tether_force((hi - r0) + lo, k));
+            v = v + f * invm * halfDt;     // end of step n
+            v = v + f * invm * halfDt;     // start of step n+1
+            r = r + cvt<double>(v) * S.dt;
+            split();
+        }
+        IO::template set_vel<Real>(S, a, v);
+        IO::template set_pos<Real>(S, a, r);
+    }
+}
+
+template <class Real, bool EXACT, class IO>
+__global__ __launch_bounds__(kStepsBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_steps(const DevSys* __restrict__ systems,
+                                                              const Tile* __restrict__ tiles, int numTiles,
+                                                              int boundaries, int flags) {
+    extern __shared__ double stash_memory[];
+    Real* stash = reinterpret_cast<Real*>(stash_memory);
+    for (int t = blockIdx.x; t < numTiles; t += gridDim.x) {
+        const Tile tile = tiles[t];
+        const DevSys& S = systems[tile.sys];
+        if (tile.kind == TILE_FREE) {
+            steps_free<Real, IO>(S, tile, boundaries, flags);
+            continue;
+        }
+        steps_bodies<Real, EXACT, IO>(S, tile, boundaries, flags, stash);
     }
 }
 
@@ -1429,13 +1646,17 @@ namespace {
 thread_local hipEvent_t t_kernelStart = nullptr, t_kernelStop = nullptr;
 
 template <class... KArgs, class... Args>
-void step_kernel(void (*kernel)(KArgs...), int grid, int block, hipStream_t stream, Args... args) {
+void step_kernel_lds(void (*kernel)(KArgs...), int grid, int block, size_t lds, hipStream_t stream, Args... args) {
     if (t_kernelStart) {
-        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, stream, t_kernelStart, t_kernelStop, 0, args...);
+        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds, stream, t_kernelStart, t_kernelStop, 0, args...);
         t_kernelStart = t_kernelStop = nullptr;
     } else {
-        kernel<<<grid, block, 0, stream>>>(args...);
+        kernel<<<grid, block, lds, stream>>>(args...);
     }
+}
+template <class... KArgs, class... Args>
+void step_kernel(void (*kernel)(KArgs...), int grid, int block, hipStream_t stream, Args... args) {
+    step_kernel_lds(kernel, grid, block, 0, stream, args...);
 }
 }  // namespace
 
@@ -1662,6 +1883,44 @@ hipError_t launch_forces(int precision, const DevSys* systems, const Tile* tiles
         else forces_for<double, SoaAtoms>(energy, grid, block, stream, systems, tiles, numTiles);
     }
     return hipGetLastError();
+}
+
+template <class IO>
+static void steps_for(int precision, int rotationMode, int grid, size_t lds, hipStream_t stream,
+                      const DevSys* systems, const Tile* tiles, int numTiles, int boundaries, int flags) {
+    auto go = [&](auto kernel) {
+        step_kernel_lds(kernel, grid, kStepsBlock, lds, stream, systems, tiles, numTiles, boundaries, flags);
+    };
+    if (precision == 0) {
+        if (rotationMode == 0) go(k_steps<float, true, IO>);
+        else go(k_steps<float, false, IO>);
+    } else {
+        if (rotationMode == 0) go(k_steps<double, true, IO>);
+        else go(k_steps<double, false, IO>);
+    }
+}
+
+size_t steps_lds_bytes(int precision, int atomsPerLane) {
+    return (size_t)kStepsBlock * ((7 * (size_t)atomsPerLane) | 1) * (precision == 0 ? sizeof(float) : sizeof(double));
+}
+
+hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
+                        int boundaries, int atomsPerLane, hipStream_t stream, int adopted) {
+    if (numTiles <= 0) return hipSuccess;
+    const size_t lds = steps_lds_bytes(precision, atomsPerLane);
+    if (lds > kStepsLdsMax) return hipErrorInvalidValue;
+    int flags = STEPS_FIRST;
+    do {
+        const int n = boundaries < kStepsPerLaunch ? boundaries : kStepsPerLaunch;
+        boundaries -= n;
+        if (boundaries == 0) flags |= STEPS_LAST;
+        if (adopted) steps_for<AdoptedAtoms>(precision, rotationMode, numTiles, lds, stream, systems, tiles, numTiles, n, flags);
+        else steps_for<SoaAtoms>(precision, rotationMode, numTiles, lds, stream, systems, tiles, numTiles, n, flags);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        flags = 0;
+    } while (boundaries > 0);
+    return hipSuccess;
 }
 
 hipError_t launch_reduce(const DevSys* systems, const int* nslots, int numSystems, int which, double* out,
