@@ -27,6 +27,7 @@
 #include "rbhip.h"
 #include "rbhip_bookkeeping.h"
 #include "rbhip_graph_cache.h"
+#include "rbhip_readback.h"
 #include "rbhip_shapes.h"
 #include "rbhip_internal.h"
 #include "rbhip_kernels.h"
@@ -741,7 +742,8 @@ struct rbhip_context {
         if (tileCache.block != blk || tileCache.lanes != lanes || tileCache.shapesVersion != shapesVersion) {
             tileCache.part = partTiles(blk, lanes);
             tileCache.force = forceTiles(blk);
-            tileCache.step = blk == kStepsBlock ? tileCache.part : partTiles(kStepsBlock, lanes);
+            // (at kStepsBlock threads the part tiles serve)
+            tileCache.step = blk == kStepsBlock ? std::vector<Tile>() : partTiles(kStepsBlock, lanes);
             validateTiles(tileCache.part, blk, maxKeSlots);
             validateTiles(tileCache.force, blk, maxPeSlots);
             validateTiles(tileCache.step, kStepsBlock, maxKeSlots);
@@ -764,7 +766,8 @@ struct rbhip_context {
         std::vector<Tile> ft = forceTiles(block);
         std::map<int, int> ones;
         std::vector<Tile> st = partTiles(setupBlock(), ones);
-        std::vector<Tile> kt = partTiles(kStepsBlock, lanes);
+        std::vector<Tile> kt;
+        if (block != kStepsBlock) kt = partTiles(kStepsBlock, lanes);
         validateTiles(kt, kStepsBlock, maxKeSlots);
         validateTiles(pt, block, maxKeSlots);
         validateTiles(ft, block, maxPeSlots);
@@ -793,7 +796,7 @@ struct rbhip_context {
         if (!kt.empty() && dStepTiles != dPartTiles)
             HIPCHK(hipMemcpyAsync(dStepTiles, kt.data(), kt.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
-        nStepTiles = (int)kt.size();
+        nStepTiles = block == kStepsBlock ? (int)pt.size() : (int)kt.size();
         nPartTiles = (int)pt.size();
         nForceTiles = (int)ft.size();
         nSetupTiles = (int)st.size();
@@ -999,8 +1002,7 @@ struct rbhip_context {
         HIPCHK(launch_stage_out(precision, dSys, dTmp, numAtoms, what, stream, layout(), dAtomOrig));
         if (what == 0 && positionsDerived && precision == RBHIP_PRECISION_MIXED && !adopted)
             HIPCHK(launch_body_atoms_out(precision, dSys, dBodyN, dBodyAtom0, numBodies, dTmp, stream, dAtomOrig));
-        HIPCHK(hipMemcpyAsync(xyz, dTmp, 3 * (size_t)numAtoms * sizeof(double), hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
+        HIPCHK(read_back(xyz, dTmp, 3 * (size_t)numAtoms * sizeof(double), device, stream));
     }
 
     // Forces replaced outside a step: momenta that carry the next step's
@@ -2455,8 +2457,7 @@ int rbhip_get_body_states(rbhip_context* ctx, double* out) {
         C.adoptedForcesIn();
         HIPCHK(launch_body_states(C.precision, C.dSys, C.dBodyN, C.dBodyAtom0, C.numBodies, C.dTmp, C.stream));
         std::vector<double> tmp(36 * (size_t)C.numBodies);
-        HIPCHK(hipMemcpyAsync(tmp.data(), C.dTmp, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, C.stream));
-        HIPCHK(hipStreamSynchronize(C.stream));
+        HIPCHK(read_back(tmp.data(), C.dTmp, tmp.size() * sizeof(double), C.device, C.stream));
         for (int ib = 0; ib < C.numBodies; ib++) {
             int r = C.internalBody[ib];
             std::memcpy(out + 36 * (size_t)r, tmp.data() + 36 * (size_t)ib, 36 * sizeof(double));
