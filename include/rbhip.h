@@ -287,9 +287,13 @@ int rbhip_part2(rbhip_context* ctx);
    trajectory as steps x [part1, forces, part2] (bit for bit in mixed
    precision, to a few ulp in FP64), without the interior steps' atom
    velocities and kinetic energies, which nothing reads.
-   Repeated sequences are replayed from HIP graphs when enabled. */
+   Where no atom's force depends on another atom (the tether alone), the
+   interior boundaries run up to 64 per launch with the state in registers.
+   Long sequences of steps with clusters or sites are replayed from a HIP
+   graph when enabled. */
 int rbhip_execute(rbhip_context* ctx, int steps);
-/* 1 = capture the repeated launches in HIP graphs and replay them (default) */
+/* 1 = capture the repeated launches of long sequences in a HIP graph and
+   replay it where that is faster (default) */
 int rbhip_use_graph(rbhip_context* ctx, int enable);
 /* 1 = fuse interior step boundaries in rbhip_execute (default), 0 = two-pass */
 int rbhip_use_fusion(rbhip_context* ctx, int enable);
@@ -377,6 +381,8 @@ int rbhip_batch_set_members(rbhip_batch* batch, int count, rbhip_context* const*
 /* launch stream of the batch (NULL = a library pool stream, the default) */
 int rbhip_batch_set_stream(rbhip_batch* batch, rbhip_stream stream);
 int rbhip_batch_set_launch(rbhip_batch* batch, int blockSize, int maxBlocks);
+/* accepted; a batch's kernels (at most two a step) are launched, which is
+   faster than replaying them */
 int rbhip_batch_use_graph(rbhip_batch* batch, int enable);
 int rbhip_batch_use_fusion(rbhip_batch* batch, int enable);
 /* steps every member `steps` times: per step one part1, one force and one

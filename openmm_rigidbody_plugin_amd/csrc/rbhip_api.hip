@@ -213,28 +213,23 @@ template <class F> hipGraphExec_t ensure_graph(GraphCache& g, const GraphKey& ke
     });
 }
 
-// The repeated launch sequences of a call, as HIP graphs: the two-pass step
-// (part1, forces, part2), one fused step boundary (fused pass, forces), and
-// kFusedChunk of those in one graph; the *Last graphs are the same steps with
-// the potential energy, which the last step of a call takes.  A graph launch
-// costs the host tens of microseconds, as much as a small system's whole
-// step, so long calls replay the chunk.
+// The repeated launch sequence of a long call, as a HIP graph: kFusedChunk
+// fused step boundaries (fused pass, forces, and any cluster and site
+// kernels).  A graph launch costs the host as much as several kernel launches
+// (one step: 33 us replayed, 24 launched; ten two-pass steps 190 and 133; 40
+// boundaries with bonds 441 and 406; 50 with clusters and sites, six kernels
+// a step, 1535 and 1564), so only whole chunks of the last kind are replayed
+// (graphPays) and everything else is launched.
 struct StepGraphs {
     static constexpr int kFusedChunk = 16;
-    enum Kind { TWO_PASS = 1, FUSED = 2, CHUNK = 3, TWO_PASS_LAST = 4, FUSED_LAST = 5 };
-    GraphCache twoPass, fused, chunk, twoPassLast, fusedLast;
-    // drops every graph (each after its stream has drained)
+    enum Kind { CHUNK = 3 };
+    GraphCache chunk;
+    // drops the graph (after its stream has drained)
     void reset() {
         HipGraphOps ops;
-        twoPass.drop(ops);
-        fused.drop(ops);
         chunk.drop(ops);
-        twoPassLast.drop(ops);
-        fusedLast.drop(ops);
     }
-    bool any() const {
-        return twoPass.valid() || fused.valid() || chunk.valid() || twoPassLast.valid() || fusedLast.valid();
-    }
+    bool any() const { return chunk.valid(); }
 };
 
 // RigidBodyIntegrator::step(steps) on a context or a batch (`o` provides the
@@ -244,8 +239,8 @@ struct StepGraphs {
 // on that atom alone, all of them before the last forces run in launches of
 // kStepsPerLaunch boundaries.  With `refine` the last step is
 // bracketed by the refined-energy kernels.  Only the last force evaluation
-// takes the potential energy (a step asks for forces alone); the graphs hold
-// the other steps, and the last one is launched on its own.
+// takes the potential energy (a step asks for forces alone); the graph holds
+// other steps only.
 template <class O> void run_steps(O& o, int steps, bool refine) {
     if (steps <= 0) return;
     const int tail = refine ? 1 : 0;
@@ -264,8 +259,8 @@ template <class O> void run_steps(O& o, int steps, bool refine) {
         o.launchPart1();
         o.launchForces(interior == 0 && !tail);
         if (interior > 0) interior--;                 // the last one below, with the energy
-        if (o.useGraph) {
-            if (interior >= StepGraphs::kFusedChunk) {
+        if constexpr (O::kGraphs) {
+            if (o.graphPays() && interior >= StepGraphs::kFusedChunk) {
                 hipGraphExec_t g = ensure_graph(o.graphs.chunk, o.graphKey(StepGraphs::CHUNK), [&] {
                     for (int i = 0; i < StepGraphs::kFusedChunk; i++) {
                         o.launchFused();
@@ -275,30 +270,14 @@ template <class O> void run_steps(O& o, int steps, bool refine) {
                 for (; interior >= StepGraphs::kFusedChunk; interior -= StepGraphs::kFusedChunk)
                     HIPCHK(hipGraphLaunch(g, o.stream));
             }
-            if (interior > 0) {
-                hipGraphExec_t g = ensure_graph(o.graphs.fused, o.graphKey(StepGraphs::FUSED), [&] {
-                    o.launchFused();
-                    o.launchForces(false);
-                });
-                for (; interior > 0; interior--) HIPCHK(hipGraphLaunch(g, o.stream));
-            }
-        } else {
-            for (; interior > 0; interior--) {
-                o.launchFused();
-                o.launchForces(false);
-            }
+        }
+        for (; interior > 0; interior--) {
+            o.launchFused();
+            o.launchForces(false);
         }
         if (steps - 1 - tail > 0) {
-            if (o.useGraph && !tail) {
-                HIPCHK(hipGraphLaunch(ensure_graph(o.graphs.fusedLast, o.graphKey(StepGraphs::FUSED_LAST), [&] {
-                                          o.launchFused();
-                                          o.launchForces(true);
-                                      }),
-                                      o.stream));
-            } else {
-                o.launchFused();
-                o.launchForces(!tail);
-            }
+            o.launchFused();
+            o.launchForces(!tail);
         }
         if (tail) {
             o.launchRefineBegin(false);
@@ -307,34 +286,10 @@ template <class O> void run_steps(O& o, int steps, bool refine) {
         }
         o.launchPart2();
     } else {
-        const int plain = steps - tail;
-        if (o.useGraph && plain > 1) {
-            hipGraphExec_t g = ensure_graph(o.graphs.twoPass, o.graphKey(StepGraphs::TWO_PASS), [&] {
-                o.launchPart1();
-                o.launchForces(false);
-                o.launchPart2();
-            });
-            for (int s = 0; s < plain - 1; s++) HIPCHK(hipGraphLaunch(g, o.stream));
-        } else {
-            for (int s = 0; s < plain - 1; s++) {
-                o.launchPart1();
-                o.launchForces(false);
-                o.launchPart2();
-            }
-        }
-        if (plain > 0) {
-            if (o.useGraph && !tail) {
-                HIPCHK(hipGraphLaunch(ensure_graph(o.graphs.twoPassLast, o.graphKey(StepGraphs::TWO_PASS_LAST), [&] {
-                                          o.launchPart1();
-                                          o.launchForces(true);
-                                          o.launchPart2();
-                                      }),
-                                      o.stream));
-            } else {
-                o.launchPart1();
-                o.launchForces(!tail);
-                o.launchPart2();
-            }
+        for (int s = 0; s < steps - tail; s++) {
+            o.launchPart1();
+            o.launchForces(!tail && s + 1 == steps);
+            o.launchPart2();
         }
         if (tail) {
             o.launchRefineBegin(true);
@@ -431,7 +386,7 @@ static size_t context_arena_bytes(size_t na, int numBodies, int numFree, int num
     b += a(3 * sizeof(double) * na) * 2;                                           // stageR, stageV
     b += a(R * na) + a(3 * R * atomStride);                                       // tether k, r0
     b += a(4 * sizeof(double) * maxKe) + a(4 * sizeof(double) * maxPe);            // partials
-    b += a(sizeof(DevSys)) + a(4 * sizeof(int)) + a(sizeof(int) * nb) * 2;
+    b += a(sizeof(DevSys)) + a(sizeof(int) * nb) * 2;
     b += a(sizeof(double) * std::max(3 * na, 36 * nb)) + a(4 * sizeof(double));  // staging, reduction
     b += a(sizeof(int) * na) * 3;                      // body index, atom index, internal order
     const size_t nc = std::max(numClasses, 1);
@@ -447,6 +402,13 @@ static size_t tile_bytes_bound(size_t na, int numBodies, int numFree, int numCla
 }
 
 // ---------------------------------------------------------------------------
+// Downloads up to this size are written to pinned memory by their kernel, the
+// larger ones copied there: 576 atoms 29 and 21 us (copied and direct), 9000
+// in order 37 and 28, 6000 shuffled 40 and 31, 36000 shuffled 79 and 79 (24-byte
+// rows in random order over the link), 72000 shuffled 137 and 162.
+constexpr size_t kDirectBytes = 256 << 10;
+static_assert(kDirectBytes <= PinnedChunks::kBytes, "a direct download fits one chunk");
+
 struct rbhip_context {
     int device = 0;
     int precision = RBHIP_PRECISION_MIXED;
@@ -512,6 +474,7 @@ struct rbhip_context {
     Tile* dForceTiles = nullptr;
     Tile* dSetupTiles = nullptr;
     Tile* dStepTiles = nullptr;                  // part tiles of kStepsBlock threads, for launchSteps
+    int atomsPerLane = 0;                        // the most body atoms a lane holds in them
     int nPartTiles = 0, nForceTiles = 0, nSetupTiles = 0, nStepTiles = 0;
     // cluster tiles, 64 clusters each: KE slots after the part tiles, and a
     // copy whose slots follow the set-up tiles
@@ -522,7 +485,6 @@ struct rbhip_context {
     static constexpr int kClusterBlock = 64;
     int maxKeSlots = 0, maxPeSlots = 0;
     int keSlots = 0;                             // slots written by the last KE producer
-    int* dSlotCounts = nullptr;                  // [0] ke, [1] pe, [2] refined ke, [3] refined pe
     int* dBodyN = nullptr;
     int* dBodyAtom0 = nullptr;
     double* dTmp = nullptr;
@@ -673,6 +635,13 @@ struct rbhip_context {
         return out;
     }
 
+    static int mostPerLane(const std::vector<Tile>& tiles) {
+        int m = 0;
+        for (const Tile& t : tiles)
+            if (t.kind == TILE_BODIES) m = std::max(m, (t.N + t.lanes - 1) / t.lanes);
+        return m;
+    }
+
     std::vector<Tile> forceTiles(int blk) const {
         std::vector<Tile> t;
         const int atomTile = FORCE_PER_THREAD * blk;
@@ -775,27 +744,27 @@ struct rbhip_context {
         // the old tables may still be read by queued work
         HIPCHK(hipStreamSynchronize(stream));
         tileArena.release();
-        dPartTiles = tileArena.allocT<Tile>(pt.size() + 1);
-        dForceTiles = tileArena.allocT<Tile>(ft.size() + 1);
-        dSetupTiles = tileArena.allocT<Tile>(st.size() + 1);
-        dStepTiles = block == kStepsBlock ? dPartTiles : tileArena.allocT<Tile>(kt.size() + 1);
         std::vector<Tile> ct = clusterTiles((int)pt.size()), cst = clusterTiles((int)st.size());
-        dClusterTiles = tileArena.allocT<Tile>(ct.size() + 1);
-        dClusterSetupTiles = tileArena.allocT<Tile>(cst.size() + 1);
-        if (!ct.empty()) {
-            HIPCHK(hipMemcpyAsync(dClusterTiles, ct.data(), ct.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
-            HIPCHK(hipMemcpyAsync(dClusterSetupTiles, cst.data(), cst.size() * sizeof(Tile), hipMemcpyHostToDevice,
-                                  stream));
-        }
-        if (!pt.empty())
-            HIPCHK(hipMemcpyAsync(dPartTiles, pt.data(), pt.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
-        if (!ft.empty())
-            HIPCHK(hipMemcpyAsync(dForceTiles, ft.data(), ft.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
-        if (!st.empty())
-            HIPCHK(hipMemcpyAsync(dSetupTiles, st.data(), st.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
-        if (!kt.empty() && dStepTiles != dPartTiles)
-            HIPCHK(hipMemcpyAsync(dStepTiles, kt.data(), kt.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
+        // one table holds them all (one allocation and one upload)
+        std::vector<Tile> all;
+        auto place = [&](const std::vector<Tile>& tiles) {
+            const size_t at = all.size();
+            all.insert(all.end(), tiles.begin(), tiles.end());
+            return at;
+        };
+        const size_t partAt = place(pt), forceAt = place(ft), setupAt = place(st), clusterAt = place(ct),
+                     clusterSetupAt = place(cst), stepAt = block == kStepsBlock ? partAt : place(kt);
+        Tile* table = tileArena.allocT<Tile>(all.size() + 1);
+        dPartTiles = table + partAt;
+        dForceTiles = table + forceAt;
+        dSetupTiles = table + setupAt;
+        dClusterTiles = table + clusterAt;
+        dClusterSetupTiles = table + clusterSetupAt;
+        dStepTiles = table + stepAt;
+        if (!all.empty())
+            HIPCHK(hipMemcpyAsync(table, all.data(), all.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
+        atomsPerLane = mostPerLane(block == kStepsBlock ? pt : kt);
         nStepTiles = block == kStepsBlock ? (int)pt.size() : (int)kt.size();
         nPartTiles = (int)pt.size();
         nForceTiles = (int)ft.size();
@@ -813,11 +782,9 @@ struct rbhip_context {
         graphs.reset();
     }
 
-    void setSlotCounts(int ke, int pe) {
-        int v[2] = {ke, pe};
-        HIPCHK(hipMemcpyAsync(dSlotCounts, v, sizeof(v), hipMemcpyHostToDevice, stream));
-        HIPCHK(hipStreamSynchronize(stream));
-    }
+    // clusters or sites make a step long enough for a graph of steps
+    static constexpr bool kGraphs = true;
+    bool graphPays() const { return useGraph && (nClusterTiles > 0 || numSites > 0); }
 
     int layout() const { return adopted ? 1 : 0; }
     // everything a captured step sequence of this context reads
@@ -868,20 +835,10 @@ struct rbhip_context {
     // no atom's force depends on another atom, and a lane's atoms fit its LDS
     bool localSteps() const {
         return !h.bondStart && numSites == 0 && numClusters == 0 &&
-               steps_lds_bytes(precision, atomsPerLane()) <= kStepsLdsMax;
-    }
-    // the most body atoms one lane holds
-    int atomsPerLane() const {
-        int m = 0;
-        for (const Class& c : classes) {
-            auto it = lanes.find(c.N);
-            const int L = it == lanes.end() ? 1 : it->second;
-            m = std::max(m, (c.N + L - 1) / L);
-        }
-        return m;
+               steps_lds_bytes(precision, atomsPerLane) <= kStepsLdsMax;
     }
     void launchSteps(int boundaries) {
-        HIPCHK(launch_steps(precision, rotationMode, dSys, dStepTiles, nStepTiles, boundaries, atomsPerLane(), stream,
+        HIPCHK(launch_steps(precision, rotationMode, dSys, dStepTiles, nStepTiles, boundaries, atomsPerLane, stream,
                             layout()));
     }
     int partKeSlots() const { return nPartTiles + nClusterTiles; }
@@ -897,12 +854,16 @@ struct rbhip_context {
     // 4 doubles reduced from the KE (which = 0), PE (1), refined KE (2) or
     // refined PE (3) partials
     void reduce(int which, double* out4) {
-        int counts[4] = {keSlots, nForceTiles, refKeSlots, nPartTiles};
-        HIPCHK(hipMemcpyAsync(dSlotCounts, counts, sizeof(counts), hipMemcpyHostToDevice, stream));
-        HIPCHK(launch_reduce(dSys, dSlotCounts + which, 1, which, dRed, stream));
-        HIPCHK(hipMemcpyAsync(hRed, dRed, 4 * sizeof(double), hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
-        for (int c = 0; c < 4; c++) out4[c] = hRed[c];
+        const int counts[4] = {keSlots, nForceTiles, refKeSlots, nPartTiles};
+        PinnedLease lease(1, stream);
+        double* sum = lease.chunks.empty() ? dRed : static_cast<double*>(lease.chunks[0]);
+        HIPCHK(launch_reduce_one(dSys, counts[which], which, sum, stream));
+        if (sum == dRed) {
+            HIPCHK(hipMemcpyAsync(hRed, dRed, 4 * sizeof(double), hipMemcpyDeviceToHost, stream));
+            sum = hRed;
+        }
+        HIPCHK(lease.wait());
+        std::memcpy(out4, sum, 4 * sizeof(double));
     }
 
     void runSetup(int geometry) {
@@ -998,11 +959,25 @@ struct rbhip_context {
     }
 
     // the state in original order: the kernels scatter through dAtomOrig
+    // (a small system's straight into pinned memory, without a copy)
+    static constexpr size_t kDirectRows = kDirectBytes / 24;
     void download(int what, double* xyz) {
-        HIPCHK(launch_stage_out(precision, dSys, dTmp, numAtoms, what, stream, layout(), dAtomOrig));
-        if (what == 0 && positionsDerived && precision == RBHIP_PRECISION_MIXED && !adopted)
-            HIPCHK(launch_body_atoms_out(precision, dSys, dBodyN, dBodyAtom0, numBodies, dTmp, stream, dAtomOrig));
-        HIPCHK(read_back(xyz, dTmp, 3 * (size_t)numAtoms * sizeof(double), device, stream));
+        const bool direct = (size_t)numAtoms <= kDirectRows;
+        PinnedLease lease(direct ? 1 : 0, stream);
+        double* rows = lease.chunks.empty() ? dTmp : static_cast<double*>(lease.chunks[0]);
+        // body atoms rebuilt from the body state are written once, by the
+        // second kernel (massless particles follow them)
+        const bool derived = what == 0 && positionsDerived && precision == RBHIP_PRECISION_MIXED && !adopted;
+        const int staged = derived && numMassless == 0 ? numFree : numAtoms;
+        HIPCHK(launch_stage_out(precision, dSys, rows, staged, what, stream, layout(), dAtomOrig));
+        if (derived)
+            HIPCHK(launch_body_atoms_out(precision, dSys, dBodyN, dBodyAtom0, numBodies, rows, stream, dAtomOrig));
+        if (rows == dTmp) {
+            HIPCHK(read_back(xyz, dTmp, 3 * (size_t)numAtoms * sizeof(double), device, stream));
+        } else {
+            HIPCHK(lease.wait());
+            std::memcpy(xyz, rows, 3 * (size_t)numAtoms * sizeof(double));
+        }
     }
 
     // Forces replaced outside a step: momenta that carry the next step's
@@ -1132,7 +1107,7 @@ struct rbhip_batch {
     int device = 0;
     hipStream_t stream = nullptr;
     int block = 256, maxBlocks = 0;
-    bool useGraph = true;
+    static constexpr bool kGraphs = false;       // two kernels a step at most: launched
     std::vector<rbhip_context*> members;
     DeviceArena arena;
     DevSys* dSystems = nullptr;
@@ -1140,16 +1115,15 @@ struct rbhip_batch {
     Tile* dForceTiles = nullptr;
     Tile* dStepTiles = nullptr;                  // as a context's, over the members
     int nPart = 0, nForce = 0, nStep = 0;
+    int atomsPerLane = 0;                        // of the step tiles, as built
     std::vector<int> memberPartTiles, memberForceTiles;
     std::vector<int> memberVersions;             // sysVersion of each member's DevSys copy
     int* dKeSlots = nullptr;
     double* dRed = nullptr;
     int precision = 0, rotationMode = 0;
     bool useFusion = true;
-    StepGraphs graphs;
 
     void rebuild() {
-        graphs.reset();
         arena.release();
         nPart = nForce = nStep = 0;
         memberPartTiles.assign(members.size(), 0);
@@ -1197,6 +1171,7 @@ struct rbhip_batch {
             HIPCHK(hipMemcpyAsync(dStepTiles, kt.data(), kt.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
         nStep = block == kStepsBlock ? (int)pt.size() : (int)kt.size();
+        atomsPerLane = rbhip_context::mostPerLane(block == kStepsBlock ? pt : kt);
         nPart = (int)pt.size();
         nForce = (int)ft.size();
     }
@@ -1216,19 +1191,6 @@ struct rbhip_batch {
         if (copied) HIPCHK(hipStreamSynchronize(stream));
     }
 
-    GraphKey graphKey(int kind) const {
-        GraphKey k;
-        k.stream = stream;
-        k.systems = dSystems;
-        k.partTiles = dPartTiles;
-        k.forceTiles = dForceTiles;
-        k.numPart = nPart;
-        k.numForce = nForce;
-        k.block = block;
-        k.maxBlocks = maxBlocks;
-        k.kind = kind;
-        return k;
-    }
     // (members hold their atoms in the library's own arrays)
     void launchPart1() {
         HIPCHK(launch_part1(precision, rotationMode, dSystems, dPartTiles, nPart, block, maxBlocks, stream, 0));
@@ -1242,19 +1204,14 @@ struct rbhip_batch {
     void launchFused() {
         HIPCHK(launch_fused(precision, rotationMode, dSystems, dPartTiles, nPart, block, maxBlocks, stream, 0));
     }
-    // as for a context, for every member at the batch's workgroup size
-    int atomsPerLane() const {
-        int m = 0;
-        for (const rbhip_context* c : members) m = std::max(m, c->atomsPerLane());
-        return m;
-    }
+    // as for a context, over every member
     bool localSteps() const {
         for (const rbhip_context* c : members)
             if (c->h.bondStart || c->numSites > 0 || c->numClusters > 0) return false;
-        return steps_lds_bytes(precision, atomsPerLane()) <= kStepsLdsMax;
+        return steps_lds_bytes(precision, atomsPerLane) <= kStepsLdsMax;
     }
     void launchSteps(int boundaries) {
-        HIPCHK(launch_steps(precision, rotationMode, dSystems, dStepTiles, nStep, boundaries, atomsPerLane(), stream,
+        HIPCHK(launch_steps(precision, rotationMode, dSystems, dStepTiles, nStep, boundaries, atomsPerLane, stream,
                             0));
     }
     void launchRefineBegin(bool folded) {
@@ -1307,7 +1264,6 @@ struct rbhip_batch {
     hipEvent_t ordering = nullptr;
 
     ~rbhip_batch() {
-        graphs.reset();
         arena.release();
         if (ordering) (void)hipEventDestroy(ordering);
     }
@@ -1582,7 +1538,6 @@ static int create_context(int numAtoms, const double* masses, const int* bodyInd
         h.kePart = C.arena.allocT<double>(4 * (size_t)C.maxKeSlots);
         h.pePart = C.arena.allocT<double>(4 * (size_t)C.maxPeSlots);
         C.dSys = C.arena.allocT<DevSys>(1);
-        C.dSlotCounts = C.arena.allocT<int>(4);
         C.dBodyN = C.arena.allocT<int>(nb);
         C.dBodyAtom0 = C.arena.allocT<int>(nb);
         C.tmpCount = std::max(3 * na, 36 * nb);
@@ -2766,7 +2721,6 @@ int rbhip_batch_set_stream(rbhip_batch* batch, rbhip_stream stream) {
         HIPCHK(hipStreamSynchronize(batch->stream));
         batch->stream = stream ? reinterpret_cast<hipStream_t>(stream) : pooled_stream(batch->device);
         batch->arena.stream = batch->stream;
-        batch->graphs.reset();
     });
 }
 
@@ -2791,8 +2745,7 @@ int rbhip_batch_set_launch(rbhip_batch* batch, int blockSize, int maxBlocks) {
 int rbhip_batch_use_graph(rbhip_batch* batch, int enable) {
     return guard([&] {
         require(batch, "null batch");
-        batch->useGraph = enable != 0;
-        if (!batch->useGraph) batch->graphs.reset();
+        (void)enable;   // (a batch's steps are launched: faster than replaying two kernels a step)
     });
 }
 
@@ -2830,8 +2783,7 @@ int rbhip_batch_kinetic_energies(rbhip_batch* batch, double* out) {
         HIPCHK(hipMemcpyAsync(batch->dKeSlots, slots.data(), n * sizeof(int), hipMemcpyHostToDevice, batch->stream));
         HIPCHK(launch_reduce(batch->dSystems, batch->dKeSlots, (int)n, 0, batch->dRed, batch->stream));
         std::vector<double> r(4 * n);
-        HIPCHK(hipMemcpyAsync(r.data(), batch->dRed, r.size() * sizeof(double), hipMemcpyDeviceToHost, batch->stream));
-        HIPCHK(hipStreamSynchronize(batch->stream));
+        HIPCHK(read_back(r.data(), batch->dRed, r.size() * sizeof(double), batch->device, batch->stream));
         for (size_t m = 0; m < n; m++) {
             out[2 * m] = 0.5 * r[4 * m];
             out[2 * m + 1] = 0.5 * r[4 * m + 1];

@@ -72,6 +72,8 @@ hipError_t launch_clusters(int precision, const DevSys* systems, const Tile* til
 // which: 0 kePart, 1 pePart, 2 refKePart, 3 refPePart
 hipError_t launch_reduce(const DevSys* systems, const int* nslots, int numSystems, int which, double* out,
                          hipStream_t stream);
+// the same for one system with nslots partials
+hipError_t launch_reduce_one(const DevSys* sys, int nslots, int which, double* out, hipStream_t stream);
 hipError_t launch_copy(const void* src, void* dst, size_t bytes, hipStream_t stream);
 
 // setup and state conversion (rbhip_setup.hip, FP64 without contraction)

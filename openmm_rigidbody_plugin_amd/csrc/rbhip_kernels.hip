@@ -1604,12 +1604,16 @@ __global__ __launch_bounds__(kStepsBlock) __attribute__((amdgpu_waves_per_eu(2))
     }
 }
 
-// deterministic sum of `nslots` 4-double partials of each system; one block per system
+// deterministic sum of the 4-double partials of each system; one block per
+// system.  nslots: their count per system, or null for `count` (one system).
+// `out` may be pinned host memory: a context's energies are written there by
+// the kernel, so a query is one launch and one wait (28 us with the count
+// copied up and the sum copied down, 13 without).
 __global__ __launch_bounds__(256) void k_reduce(const DevSys* __restrict__ systems, const int* __restrict__ nslots,
-                                                 int which, double* __restrict__ out) {
+                                                 int count, int which, double* __restrict__ out) {
     const DevSys& S = systems[blockIdx.x];
     const double* part = which == 0 ? S.kePart : which == 1 ? S.pePart : which == 2 ? S.refKePart : S.refPePart;
-    int n = nslots[blockIdx.x];
+    int n = nslots ? nslots[blockIdx.x] : count;
     __shared__ double red[256][4];
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int s = threadIdx.x; s < n; s += blockDim.x)
@@ -1926,7 +1930,12 @@ hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, 
 hipError_t launch_reduce(const DevSys* systems, const int* nslots, int numSystems, int which, double* out,
                          hipStream_t stream) {
     if (numSystems <= 0) return hipSuccess;
-    k_reduce<<<numSystems, 256, 0, stream>>>(systems, nslots, which, out);
+    k_reduce<<<numSystems, 256, 0, stream>>>(systems, nslots, 0, which, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_reduce_one(const DevSys* sys, int nslots, int which, double* out, hipStream_t stream) {
+    k_reduce<<<1, 256, 0, stream>>>(sys, nullptr, nslots, which, out);
     return hipGetLastError();
 }
 

@@ -59,11 +59,22 @@ private:
     int made_ = 0;
 };
 
-// chunks held for the length of a scope
+// chunks held for the length of a scope; work that writes them is waited for
+// (wait, or on the way out of a scope left early) before they are put back
 struct PinnedLease {
     std::vector<void*> chunks;
-    explicit PinnedLease(int want) : chunks(PinnedChunks::get().take(want)) {}
-    ~PinnedLease() { PinnedChunks::get().put(chunks); }
+    hipStream_t pending;   // work queued here may still write the chunks
+    explicit PinnedLease(int want, hipStream_t writer = nullptr)
+        : chunks(PinnedChunks::get().take(want)), pending(writer) {}
+    ~PinnedLease() {
+        if (pending) (void)hipStreamSynchronize(pending);
+        PinnedChunks::get().put(chunks);
+    }
+    hipError_t wait() {
+        hipStream_t s = pending;
+        pending = nullptr;
+        return hipStreamSynchronize(s);
+    }
     PinnedLease(const PinnedLease&) = delete;
     PinnedLease& operator=(const PinnedLease&) = delete;
 };
