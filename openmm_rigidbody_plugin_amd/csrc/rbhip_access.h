@@ -69,33 +69,52 @@ template <class Real> __device__ __forceinline__ void store_pos(const DevSys& S,
 // ---------------------------------------------------------------------------
 // Where the step kernels find the atom state.  Both policies give the same
 // values to the same arithmetic, so a trajectory does not depend on the
-// layout (given forces both layouts represent exactly).
+// layout (given forces both layouts represent exactly).  at(i) is where atom i
+// lies; the ..._at forms take it, so that a body's places can be read before
+// its first store (a load behind a store to memory that it may alias waits
+// for the store to be on its way, and then for a round trip of its own).
 // ---------------------------------------------------------------------------
 // the library's own component-major arrays (internal atom order)
 struct SoaAtoms {
     static constexpr bool adopted = false;
-    template <class Real> static __device__ __forceinline__ V3<Real> force(const DevSys& S, int i) {
+    static __device__ __forceinline__ int at(const DevSys&, int i) { return i; }
+    template <class Real> static __device__ __forceinline__ V3<Real> force_at(const DevSys& S, int i) {
         return ld3<Real>(S.force, S.atomStride, i);
+    }
+    template <class Real> static __device__ __forceinline__ V3<Real> force(const DevSys& S, int i) {
+        return force_at<Real>(S, i);
     }
     // a force as the array holds it
     template <class Real> static __device__ __forceinline__ V3<Real> held_force(V3<Real> f) { return f; }
     // FP64 position of a free atom (hi + lo in mixed precision)
-    template <class Real> static __device__ __forceinline__ V3<double> pos(const DevSys& S, int i) {
+    template <class Real> static __device__ __forceinline__ V3<double> pos_at(const DevSys& S, int i) {
         return load_pos<Real>(S, i);
     }
-    template <class Real> static __device__ __forceinline__ void set_pos(const DevSys& S, int i, V3<double> p) {
+    template <class Real> static __device__ __forceinline__ V3<double> pos(const DevSys& S, int i) {
+        return pos_at<Real>(S, i);
+    }
+    template <class Real> static __device__ __forceinline__ void set_pos_at(const DevSys& S, int i, V3<double> p) {
         store_pos<Real>(S, i, p);
+    }
+    template <class Real> static __device__ __forceinline__ void set_pos(const DevSys& S, int i, V3<double> p) {
+        set_pos_at<Real>(S, i, p);
     }
     // a body atom keeps its device-precision position only: its exact value
     // is r_cm + A(q)^T d, rebuilt when positions are read back
-    template <class Real> static __device__ __forceinline__ void set_body_pos(const DevSys& S, int i, V3<double> p) {
+    template <class Real> static __device__ __forceinline__ void set_body_pos_at(const DevSys& S, int i, V3<double> p) {
         st3<Real>(S.pos, S.atomStride, i, cvt<Real>(p));
     }
-    template <class Real> static __device__ __forceinline__ V3<Real> vel(const DevSys& S, int i) {
+    template <class Real> static __device__ __forceinline__ V3<Real> vel_at(const DevSys& S, int i) {
         return ld3<Real>(S.vel, S.atomStride, i);
     }
-    template <class Real> static __device__ __forceinline__ void set_vel(const DevSys& S, int i, V3<Real> v) {
+    template <class Real> static __device__ __forceinline__ V3<Real> vel(const DevSys& S, int i) {
+        return vel_at<Real>(S, i);
+    }
+    template <class Real> static __device__ __forceinline__ void set_vel_at(const DevSys& S, int i, V3<Real> v) {
         st3<Real>(S.vel, S.atomStride, i, v);
+    }
+    template <class Real> static __device__ __forceinline__ void set_vel(const DevSys& S, int i, V3<Real> v) {
+        set_vel_at<Real>(S, i, v);
     }
 };
 
@@ -104,11 +123,15 @@ struct SoaAtoms {
 // fixed-point force array; w components are never written
 struct AdoptedAtoms {
     static constexpr bool adopted = true;
-    template <class Real> static __device__ __forceinline__ V3<Real> force(const DevSys& S, int i) {
-        const long long* f = S.ommForce + S.ommSlot[i];
+    static __device__ __forceinline__ int at(const DevSys& S, int i) { return S.ommSlot[i]; }
+    template <class Real> static __device__ __forceinline__ V3<Real> force_at(const DevSys& S, int s) {
+        const long long* f = S.ommForce + s;
         const size_t st = (size_t)S.ommStride;
         const double u = 1.0 / kFixedPointScale;
         return {(Real)((double)f[0] * u), (Real)((double)f[st] * u), (Real)((double)f[2 * st] * u)};
+    }
+    template <class Real> static __device__ __forceinline__ V3<Real> force(const DevSys& S, int i) {
+        return force_at<Real>(S, at(S, i));
     }
     // a force as the fixed-point array holds it (OpenMM's conversion:
     // truncation of f * 2^32)
@@ -118,8 +141,7 @@ struct AdoptedAtoms {
         return {(Real)((double)fixed_point((double)f.x) * u), (Real)((double)fixed_point((double)f.y) * u),
                 (Real)((double)fixed_point((double)f.z) * u)};
     }
-    template <class Real> static __device__ __forceinline__ V3<double> pos(const DevSys& S, int i) {
-        const int s = S.ommSlot[i];
+    template <class Real> static __device__ __forceinline__ V3<double> pos_at(const DevSys& S, int s) {
         Q4<Real> p = ld4<Real>(S.ommPosq, s);
         V3<double> r = {(double)p.a, (double)p.b, (double)p.c};
         if (sizeof(Real) == 4) {
@@ -130,8 +152,10 @@ struct AdoptedAtoms {
         }
         return r;
     }
-    template <class Real> static __device__ __forceinline__ void set_pos(const DevSys& S, int i, V3<double> p) {
-        const int s = S.ommSlot[i];
+    template <class Real> static __device__ __forceinline__ V3<double> pos(const DevSys& S, int i) {
+        return pos_at<Real>(S, at(S, i));
+    }
+    template <class Real> static __device__ __forceinline__ void set_pos_at(const DevSys& S, int s, V3<double> p) {
         Real* q = reinterpret_cast<Real*>(S.ommPosq) + 4 * (size_t)s;
         if (sizeof(Real) == 4) {
             float* c = S.ommPosqCorr + 4 * (size_t)s;
@@ -144,18 +168,27 @@ struct AdoptedAtoms {
             q[0] = (Real)p.x; q[1] = (Real)p.y; q[2] = (Real)p.z;
         }
     }
+    template <class Real> static __device__ __forceinline__ void set_pos(const DevSys& S, int i, V3<double> p) {
+        set_pos_at<Real>(S, at(S, i), p);
+    }
     // OpenMM's force kernels read posq (and the correction), so body atoms
     // are stored at full precision like free atoms
-    template <class Real> static __device__ __forceinline__ void set_body_pos(const DevSys& S, int i, V3<double> p) {
-        set_pos<Real>(S, i, p);
+    template <class Real> static __device__ __forceinline__ void set_body_pos_at(const DevSys& S, int s, V3<double> p) {
+        set_pos_at<Real>(S, s, p);
     }
-    template <class Real> static __device__ __forceinline__ V3<Real> vel(const DevSys& S, int i) {
-        const double* v = S.ommVelm + 4 * (size_t)S.ommSlot[i];
+    template <class Real> static __device__ __forceinline__ V3<Real> vel_at(const DevSys& S, int s) {
+        const double* v = S.ommVelm + 4 * (size_t)s;
         return {(Real)v[0], (Real)v[1], (Real)v[2]};
     }
-    template <class Real> static __device__ __forceinline__ void set_vel(const DevSys& S, int i, V3<Real> v) {
-        double* o = S.ommVelm + 4 * (size_t)S.ommSlot[i];
+    template <class Real> static __device__ __forceinline__ V3<Real> vel(const DevSys& S, int i) {
+        return vel_at<Real>(S, at(S, i));
+    }
+    template <class Real> static __device__ __forceinline__ void set_vel_at(const DevSys& S, int s, V3<Real> v) {
+        double* o = S.ommVelm + 4 * (size_t)s;
         o[0] = (double)v.x; o[1] = (double)v.y; o[2] = (double)v.z;
+    }
+    template <class Real> static __device__ __forceinline__ void set_vel(const DevSys& S, int i, V3<Real> v) {
+        set_vel_at<Real>(S, at(S, i), v);
     }
 };
 

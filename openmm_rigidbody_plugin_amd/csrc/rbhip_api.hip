@@ -457,7 +457,15 @@ struct rbhip_context {
     struct Class { int N, firstBody, count, firstAtom, shapes = 0; };
     std::vector<Class> classes;
     std::map<int, int> lanes;                    // atoms per body -> lanes per body
-    int block = 256, maxBlocks = 0;
+    // One wave per workgroup: the FP64 exact rotation is register heavy, and
+    // on adopted arrays, whose scattered accesses are bound by each CU's
+    // address rate, one-wave workgroups spread evenly (part 1, forces, part 2
+    // with 64, 128, 256 and 512 threads: 100k waters 11.6/10.5/13.3,
+    // 13.0/11.5/13.9, 16.5/13.4/15.8 and 27.8/14.8/19.6 us; 10k waters
+    // 6.2/4.8/5.8 with 64, 10.8/7.6/9.5 with 256; 400k 31.6/31.4/43.4 and
+    // 35.4/33.2/45.3).  The library's own arrays run alike with 64 and 256
+    // (1M waters: 31.8/16.3/30.5 and 31.6/16.1/30.9).
+    int block = 64, maxBlocks = 0;
     // bodies of one shape share body-fixed coordinate rows (mixed precision)
     static constexpr int kMaxShapes = 8, kShapeSample = 32, kShareMinBodies = 64;
     bool shareFramesOn = true;                   // rbhip_set_shared_frames
@@ -1492,7 +1500,6 @@ static int create_context(int numAtoms, const double* masses, const int* bodyInd
         }
 
         // ---- device allocation ----
-        if (rotationMode == 0) C.block = 64;   // the FP64 exact rotation is register heavy
         const size_t R = C.realSize();
         const size_t nb = std::max(C.numBodies, 1);
         DevSys& h = C.h;

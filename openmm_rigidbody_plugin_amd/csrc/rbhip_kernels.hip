@@ -89,6 +89,20 @@ template <class Real> __device__ __forceinline__ Body<Real> load_body(const DevS
 // more than 6 atoms, several lanes each)
 constexpr int STRIDED_BATCH = 8;
 
+// Adopted arrays lie in their caller's order, so a wave's accesses to them are
+// scattered, and a loop over a lane's atoms waits for a round trip per atom,
+// behind the stores of the atom before (which may alias).  So a lane loads
+// several atoms before it stores any.  How many, for the atoms' forces: 4 in
+// mixed precision (100k waters 10.5 -> 9.1 us), 2 in double (40k waters 6.6 ->
+// 6.2; 4: 6.9).  For free atoms in the step kernels: 4 in mixed precision
+// (300k free atoms, part 1 41.2 -> 37.4 us), 1 in double, where the registers
+// of 4 cost bodies in the same launch more (20k mixed bodies and 30k free
+// atoms, exact, part 1: 8.8 us, with 4 9.3; 300k free atoms 32.2, with 4
+// 29.9).  The library's own arrays, whose accesses are coalesced, gain nothing
+// from a batch.
+template <class Real, class IO> constexpr int force_batch() { return !IO::adopted ? 1 : sizeof(Real) == 4 ? 4 : 2; }
+template <class Real, class IO> constexpr int free_batch() { return IO::adopted && sizeof(Real) == 4 ? 4 : 1; }
+
 // A(q)^T d of atom u of a lane's batch.  (The first of a batch rounds its y
 // product and the others their x product, as the compiler fused them when
 // these loops were tuned; one rule for all kernels keeps their trajectories
@@ -179,31 +193,41 @@ __device__ __forceinline__ void body_sums_any(const DevSys& S, const Rot<Real>& 
 }
 
 // atom positions r_cm + A(q)^T d_j: fp32 in mixed precision (the force field's
-// view; the exact value is rebuilt from the body state on download)
+// view; the exact value is rebuilt from the body state on download).  Bodies
+// of 2 and 3 atoms, which lie in a plane of their principal axes, are placed
+// with the y products rounded, as part 1 always placed them in adopted arrays,
+// which show the last bit of the offset.
 template <class Real, bool EXACT, int NC, class IO>
 __device__ __forceinline__ void body_positions(const DevSys& S, const Rot<Real>& R, V3<double> rc, int atom0,
                                                int dbase, int N, int sub, int lanes) {
     if constexpr (NC > 0) {
         V3<Real> dj[NC];
+        int at[NC];
 #pragma unroll
-        for (int j = 0; j < NC; j++) dj[j] = ld3<Real>(S.d, S.dStride, dbase + j);
+        for (int j = 0; j < NC; j++) {
+            dj[j] = ld3<Real>(S.d, S.dStride, dbase + j);
+            at[j] = IO::at(S, atom0 + j);
+        }
 #pragma unroll
         for (int j = 0; j < NC; j++)
-            IO::template set_body_pos<Real>(S, atom0 + j,
-                                            rc + cvt<double>(place_apply<(!EXACT && NC <= 4)>(R, dj[j])));
+            IO::template set_body_pos_at<Real>(S, at[j],
+                                               rc + cvt<double>(place_apply<(!EXACT && NC == 4)>(R, dj[j])));
     } else {
         // loads of a batch first, then its stores (one round trip per batch)
         constexpr int U = STRIDED_BATCH;
         for (int j0 = sub; j0 < N; j0 += U * lanes) {
             V3<Real> dj[U];
+            int at[U];
 #pragma unroll
             for (int u = 0; u < U; u++)
-                if (j0 + u * lanes < N) dj[u] = ld3<Real>(S.d, S.dStride, dbase + j0 + u * lanes);
+                if (j0 + u * lanes < N) {
+                    dj[u] = ld3<Real>(S.d, S.dStride, dbase + j0 + u * lanes);
+                    at[u] = IO::at(S, atom0 + j0 + u * lanes);
+                }
 #pragma unroll
             for (int u = 0; u < U; u++)
                 if (j0 + u * lanes < N)
-                    IO::template set_body_pos<Real>(S, atom0 + j0 + u * lanes,
-                                                    rc + cvt<double>(strided_apply(R, dj[u], u)));
+                    IO::template set_body_pos_at<Real>(S, at[u], rc + cvt<double>(strided_apply(R, dj[u], u)));
         }
     }
 }
@@ -224,30 +248,44 @@ __device__ __forceinline__ void body_positions_any(const DevSys& S, const Rot<Re
     }
 }
 
+// v_cm + w x delta with its fused operations written out
+template <class Real> __device__ __forceinline__ V3<Real> atom_velocity(V3<Real> vcm, V3<Real> ws, V3<Real> dl) {
+    return {vcm.x + fma(ws.y, dl.z, -(ws.z * dl.y)), vcm.y + fma(ws.z, dl.x, -(ws.x * dl.z)),
+            vcm.z + fma(ws.x, dl.y, -(ws.y * dl.x))};
+}
+
 template <class Real, int NC, class IO>
 __device__ __forceinline__ void body_velocities(const DevSys& S, const Rot<Real>& R, V3<Real> vcm, V3<Real> ws,
                                                 int atom0, int dbase, int N, int sub, int lanes) {
     if constexpr (NC > 0) {
+        V3<Real> dj[NC];
+        int at[NC];
 #pragma unroll
         for (int j = 0; j < NC; j++) {
-            V3<Real> dl = apply(R, ld3<Real>(S.d, S.dStride, dbase + j));
-            IO::template set_vel<Real>(S, atom0 + j, vcm + cross(ws, dl));
+            dj[j] = ld3<Real>(S.d, S.dStride, dbase + j);
+            at[j] = IO::at(S, atom0 + j);
         }
+#pragma unroll
+        for (int j = 0; j < NC; j++)
+            IO::template set_vel_at<Real>(S, at[j], atom_velocity(vcm, ws, step_apply<true>(R, dj[j])));
     } else {
         constexpr int U = STRIDED_BATCH;
         for (int j0 = sub; j0 < N; j0 += U * lanes) {
             V3<Real> dj[U];
+            int at[U];
 #pragma unroll
             for (int u = 0; u < U; u++)
-                if (j0 + u * lanes < N) dj[u] = ld3<Real>(S.d, S.dStride, dbase + j0 + u * lanes);
+                if (j0 + u * lanes < N) {
+                    dj[u] = ld3<Real>(S.d, S.dStride, dbase + j0 + u * lanes);
+                    at[u] = IO::at(S, atom0 + j0 + u * lanes);
+                }
 #pragma unroll
             for (int u = 0; u < U; u++)
                 if (j0 + u * lanes < N)
-                    IO::template set_vel<Real>(S, atom0 + j0 + u * lanes, vcm + cross(ws, apply(R, dj[u])));
+                    IO::template set_vel_at<Real>(S, at[u], atom_velocity(vcm, ws, strided_apply(R, dj[u], u)));
         }
     }
 }
-
 // A(q) x from the rows of A(q)^T, fused operations written out as in
 // step_apply: the y product rounded, or the x product for the bodies whose
 // NO-SQUISH fused pass keeps them in registers (one lane, 2 to 4 atoms)
@@ -317,34 +355,58 @@ template <class Real> __device__ __forceinline__ V3<double> load_rcm(const DevSy
 // part 1
 // ---------------------------------------------------------------------------
 // free-atom tiles hold up to FREE_PER_THREAD atoms per thread (strided by
-// the workgroup size, so each pass over the tile is coalesced)
+// the workgroup size, so each pass over the tile is coalesced): load(u, a) for
+// U of a thread's atoms, then use(u, a) for them
+template <int U, class Load, class Use>
+__device__ __forceinline__ void over_tile(const Tile& tile, Load&& load, Use&& use) {
+    const int step = blockDim.x;
+    for (int i0 = threadIdx.x; i0 < tile.count; i0 += U * step) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i0 + u * step < tile.count) load(u, tile.first + i0 + u * step);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i0 + u * step < tile.count) use(u, tile.first + i0 + u * step);
+    }
+}
+// a batch of free atoms as a step reads them
+template <class Real, class IO, int U> struct FreeBatch {
+    int at[U];
+    V3<Real> v[U], f[U];
+    Real invm[U];
+    __device__ __forceinline__ void load(const DevSys& S, int u, int a) {
+        at[u] = IO::at(S, a);
+        v[u] = IO::template vel_at<Real>(S, at[u]);
+        f[u] = IO::template force_at<Real>(S, at[u]);
+        invm[u] = reinterpret_cast<const Real*>(S.freeInvM)[a];
+    }
+};
+
 template <class Real, class IO>
 __device__ __forceinline__ void part1_free(const DevSys& S, const Tile& tile) {
-    Real halfDt = (Real)(0.5 * S.dt);
-    for (int i = threadIdx.x; i < tile.count; i += blockDim.x) {
-        int a = tile.first + i;
-        V3<Real> v = IO::template vel<Real>(S, a);
-        V3<Real> f = IO::template force<Real>(S, a);
-        Real invm = reinterpret_cast<const Real*>(S.freeInvM)[a];
-        v = v + f * invm * halfDt;
-        V3<double> r = IO::template pos<Real>(S, a);
+    const Real halfDt = (Real)(0.5 * S.dt);
+    constexpr int U = free_batch<Real, IO>();
+    FreeBatch<Real, IO, U> atoms;
+    V3<double> r[U];
+    over_tile<U>(tile, [&](int u, int a) {
+        atoms.load(S, u, a);
+        r[u] = IO::template pos_at<Real>(S, atoms.at[u]);
+    }, [&](int u, int a) {
+        V3<Real> v = atoms.v[u] + atoms.f[u] * atoms.invm[u] * halfDt;
+        V3<double> x = r[u] + cvt<double>(v) * S.dt;
         if constexpr (IO::adopted) {
             if (S.posDelta) {
                 // the caller's constrained displacement; the correction to
                 // the unconstrained drift waits for part 2
-                const double* pd = S.posDelta + 4 * (size_t)S.ommSlot[a];
-                V3<double> ru = r + cvt<double>(v) * S.dt;
-                r = r + V3<double>{pd[0], pd[1], pd[2]};
-                st3<Real>(S.freeCorr, S.numFree, a, cvt<Real>(r - ru));
-                IO::template set_vel<Real>(S, a, v);
-                IO::template set_pos<Real>(S, a, r);
-                continue;
+                const double* pd = S.posDelta + 4 * (size_t)atoms.at[u];
+                const V3<double> ru = x;
+                x = r[u] + V3<double>{pd[0], pd[1], pd[2]};
+                st3<Real>(S.freeCorr, S.numFree, a, cvt<Real>(x - ru));
             }
         }
-        r = r + cvt<double>(v) * S.dt;
-        IO::template set_vel<Real>(S, a, v);
-        IO::template set_pos<Real>(S, a, r);
-    }
+        IO::template set_vel_at<Real>(S, atoms.at[u], v);
+        IO::template set_pos_at<Real>(S, atoms.at[u], x);
+    });
 }
 
 // The free atoms' drift displacements (v + F (1/m) dt/2) dt, as part 1
@@ -382,12 +444,13 @@ __device__ __forceinline__ void part1_bodies(const DevSys& S, const Tile& tile) 
     Body<Real> B = load_body<Real>(S, k, sh.ks);
     V3<double> rc = load_rcm<Real>(S, k);
     drift_and_rotate<Real, EXACT>(S, B, rc);
+    body_positions_any<Real, EXACT, IO>(S, step_rot(B.q), rc, atom0, dbase, tile.N, sub, tile.lanes);
+    // (last: loads behind these stores would wait for them)
     if (sub == 0) {
         st4<Real>(S.q, k, B.q);
         stp3<Real>(S.L, k, B.L);
         store_rcm<Real>(S, k, rc);
     }
-    body_positions_any<Real, EXACT, IO>(S, step_rot(B.q), rc, atom0, dbase, tile.N, sub, tile.lanes);
 }
 
 // How a step kernel holds its system descriptor.  The exact-rotation kernels
@@ -416,19 +479,17 @@ __global__ __launch_bounds__(EXACT ? 256 : 512) void k_part1(const DevSys* __res
 // ---------------------------------------------------------------------------
 template <class Real, class IO>
 __device__ __forceinline__ void part2_free(const DevSys& S, const Tile& tile, double (&ke)[2]) {
-    Real halfDt = (Real)(0.5 * S.dt);
-    for (int i = threadIdx.x; i < tile.count; i += blockDim.x) {
-        int a = tile.first + i;
-        V3<Real> v = IO::template vel<Real>(S, a);
-        V3<Real> f = IO::template force<Real>(S, a);
-        Real invm = reinterpret_cast<const Real*>(S.freeInvM)[a];
-        v = v + f * invm * halfDt;
+    const Real halfDt = (Real)(0.5 * S.dt);
+    constexpr int U = free_batch<Real, IO>();
+    FreeBatch<Real, IO, U> atoms;
+    over_tile<U>(tile, [&](int u, int a) { atoms.load(S, u, a); }, [&](int u, int a) {
+        V3<Real> v = atoms.v[u] + atoms.f[u] * atoms.invm[u] * halfDt;
         // (R - saved) / dt of a constrained part 1
         if (IO::adopted && S.corrPending) v = v + ld3<Real>(S.freeCorr, S.numFree, a) * (Real)(1.0 / S.dt);
-        IO::template set_vel<Real>(S, a, v);
+        IO::template set_vel_at<Real>(S, atoms.at[u], v);
         V3<double> vd = cvt<double>(v);
-        ke[0] += dot(vd, vd) / (double)invm;
-    }
+        ke[0] += dot(vd, vd) / (double)atoms.invm[u];
+    });
 }
 
 template <class Real, class IO>
@@ -453,13 +514,13 @@ __device__ __forceinline__ void part2_bodies(const DevSys& S, const Tile& tile, 
     V3<double> L = kicked(cvt<double>(B.L), tb, halfDt);
     V3<double> w = hadamard(cvt<double>(B.invI), L);
     V3<double> vcm = p * (double)B.invM;
-    V3<Real> ws = apply(R, cvt<Real>(w));
+    const V3<Real> ws = step_apply<true>(R, cvt<Real>(w)), vc = cvt<Real>(vcm);
     switch (tile.lanes == 1 ? N : 0) {
-    case 2: body_velocities<Real, 2, IO>(S, R, cvt<Real>(vcm), ws, atom0, dbase, N, 0, 1); break;
-    case 3: body_velocities<Real, 3, IO>(S, R, cvt<Real>(vcm), ws, atom0, dbase, N, 0, 1); break;
-    case 4: body_velocities<Real, 4, IO>(S, R, cvt<Real>(vcm), ws, atom0, dbase, N, 0, 1); break;
-    case 6: body_velocities<Real, 6, IO>(S, R, cvt<Real>(vcm), ws, atom0, dbase, N, 0, 1); break;
-    default: body_velocities<Real, 0, IO>(S, R, cvt<Real>(vcm), ws, atom0, dbase, N, sub, tile.lanes); break;
+    case 2: body_velocities<Real, 2, IO>(S, R, vc, ws, atom0, dbase, N, 0, 1); break;
+    case 3: body_velocities<Real, 3, IO>(S, R, vc, ws, atom0, dbase, N, 0, 1); break;
+    case 4: body_velocities<Real, 4, IO>(S, R, vc, ws, atom0, dbase, N, 0, 1); break;
+    case 6: body_velocities<Real, 6, IO>(S, R, vc, ws, atom0, dbase, N, 0, 1); break;
+    default: body_velocities<Real, 0, IO>(S, R, vc, ws, atom0, dbase, N, sub, tile.lanes); break;
     }
     if (sub == 0) {
         ke[0] = dot(p, vcm);
@@ -495,19 +556,20 @@ __global__ __launch_bounds__(512) void k_part2(const DevSys* __restrict__ system
 // ---------------------------------------------------------------------------
 template <class Real, class IO>
 __device__ __forceinline__ void fused_free(const DevSys& S, const Tile& tile) {
-    Real halfDt = (Real)(0.5 * S.dt);
-    for (int i = threadIdx.x; i < tile.count; i += blockDim.x) {
-        int a = tile.first + i;
-        V3<Real> v = IO::template vel<Real>(S, a);
-        V3<Real> f = IO::template force<Real>(S, a);
-        Real invm = reinterpret_cast<const Real*>(S.freeInvM)[a];
-        v = v + f * invm * halfDt;     // end of step n
-        v = v + f * invm * halfDt;     // start of step n+1
-        V3<double> r = IO::template pos<Real>(S, a);
-        r = r + cvt<double>(v) * S.dt;
-        IO::template set_vel<Real>(S, a, v);
-        IO::template set_pos<Real>(S, a, r);
-    }
+    const Real halfDt = (Real)(0.5 * S.dt);
+    constexpr int U = free_batch<Real, IO>();
+    FreeBatch<Real, IO, U> atoms;
+    V3<double> r[U];
+    over_tile<U>(tile, [&](int u, int a) {
+        atoms.load(S, u, a);
+        r[u] = IO::template pos_at<Real>(S, atoms.at[u]);
+    }, [&](int u, int) {
+        V3<Real> v = atoms.v[u];
+        v = v + atoms.f[u] * atoms.invm[u] * halfDt;     // end of step n
+        v = v + atoms.f[u] * atoms.invm[u] * halfDt;     // start of step n+1
+        IO::template set_vel_at<Real>(S, atoms.at[u], v);
+        IO::template set_pos_at<Real>(S, atoms.at[u], r[u] + cvt<double>(v) * S.dt);
+    });
 }
 
 // part2 of step n and the first half-kick of step n+1 on the body momenta
@@ -537,10 +599,12 @@ __device__ __forceinline__ void fused_body_regs(const DevSys& S, int k, int atom
     Body<Real> B = load_body<Real>(S, k, ks);
     V3<double> rc = load_rcm<Real>(S, k);
     V3<Real> dj[NC], fj[NC];
+    int at[NC];
 #pragma unroll
     for (int j = 0; j < NC; j++) {
         dj[j] = ld3<Real>(S.d, S.dStride, dbase + j);
-        fj[j] = IO::template force<Real>(S, atom0 + j);
+        at[j] = IO::at(S, atom0 + j);
+        fj[j] = IO::template force_at<Real>(S, at[j]);
     }
     Rot<Real> R = step_rot(B.q);
     V3<double> F = {0.0, 0.0, 0.0}, tau = {0.0, 0.0, 0.0};
@@ -557,7 +621,7 @@ __device__ __forceinline__ void fused_body_regs(const DevSys& S, int k, int atom
     Rot<Real> R1 = step_rot(B.q);
 #pragma unroll
     for (int j = 0; j < NC; j++)
-        IO::template set_body_pos<Real>(S, atom0 + j, rc + cvt<double>(place_apply<!EXACT>(R1, dj[j])));
+        IO::template set_body_pos_at<Real>(S, at[j], rc + cvt<double>(place_apply<!EXACT>(R1, dj[j])));
 }
 
 template <class Real, bool EXACT, class IO>
@@ -590,8 +654,8 @@ __device__ __forceinline__ void fused_bodies(const DevSys& S, const Tile& tile) 
     if (!active) return;
     fused_kicks<Real>(S, B, R, F, tau, small_body(S, N, tile.lanes));
     drift_and_rotate<Real, EXACT>(S, B, rc);
-    if (sub == 0) store_body<Real>(S, k, B, rc);
     body_positions_any<Real, EXACT, IO>(S, step_rot(B.q), rc, atom0, dbase, N, sub, tile.lanes);
+    if (sub == 0) store_body<Real>(S, k, B, rc);
 }
 
 template <class Real, bool EXACT, class IO>
@@ -1229,10 +1293,9 @@ __global__ __launch_bounds__(256) void k_clusters(const DevSys* __restrict__ sys
 // body atoms (and the massless particles after them) at their fp32
 // positions in mixed precision (lo = 0), free atoms at hi + lo
 template <class Real, class IO = SoaAtoms>
-__device__ __forceinline__ void field_pos_parts(const DevSys& S, int i, V3<Real>& hi, V3<Real>& lo) {
+__device__ __forceinline__ void field_pos_parts(const DevSys& S, int i, int s, V3<Real>& hi, V3<Real>& lo) {
     lo = {(Real)0, (Real)0, (Real)0};
     if constexpr (IO::adopted) {
-        const int s = S.ommSlot[i];
         Q4<Real> p = ld4<Real>(S.ommPosq, s);
         hi = {p.a, p.b, p.c};
         if (sizeof(Real) == 4 && i < S.numFree) {
@@ -1246,19 +1309,19 @@ __device__ __forceinline__ void field_pos_parts(const DevSys& S, int i, V3<Real>
 }
 template <class Real, class IO = SoaAtoms> __device__ __forceinline__ V3<double> force_pos(const DevSys& S, int i) {
     V3<Real> hi, lo;
-    field_pos_parts<Real, IO>(S, i, hi, lo);
+    field_pos_parts<Real, IO>(S, i, IO::at(S, i), hi, lo);
     return cvt<double>(hi) + cvt<double>(lo);
 }
 // a force into the library's array, or into the adopted fixed-point array
-template <class Real, class IO> __device__ __forceinline__ void store_force(const DevSys& S, int i, V3<Real> f) {
+template <class Real, class IO> __device__ __forceinline__ void store_force(const DevSys& S, int at, V3<Real> f) {
     if constexpr (IO::adopted) {
-        long long* o = S.ommForce + S.ommSlot[i];
+        long long* o = S.ommForce + at;
         const size_t st = (size_t)S.ommStride;
         o[0] = IO::fixed_point((double)f.x);
         o[st] = IO::fixed_point((double)f.y);
         o[2 * st] = IO::fixed_point((double)f.z);
     } else {
-        st3<Real>(S.force, S.atomStride, i, f);
+        st3<Real>(S.force, S.atomStride, at, f);
     }
 }
 
@@ -1387,36 +1450,56 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
         // waits for the atom loads in flight)
         const DevSys S = systems[tile.sys];
         double e[1] = {0.0};
-        for (int i = threadIdx.x; i < tile.count; i += blockDim.x) {
-            int a = tile.first + i;
-            V3<Real> f = {(Real)0, (Real)0, (Real)0};
-            if (S.tetherScale != 0.0) {
-                Real k = S.tetherUniform ? (Real)S.tetherK0 : reinterpret_cast<const Real*>(S.tetherK)[a];
-                V3<Real> ph, pl;
-                field_pos_parts<Real, IO>(S, a, ph, pl);
-                V3<Real> dx = (ph - ld3<Real>(S.r0, S.atomStride, a)) + pl;
-                f = tether_force(dx, k);
-                if (ENERGY) {
-                    V3<double> dd = cvt<double>(dx);
-                    e[0] += 0.5 * (double)k * dot(dd, dd);
-                }
-            }
-            if (S.bondStart) {
-                int e0 = S.bondStart[a], e1 = S.bondStart[a + 1];
-                if (e0 < e1) {
-                    V3<double> pa = force_pos<Real, IO>(S, a);
-                    V3<double> fd = cvt<double>(f);
-                    for (int b = e0; b < e1; b++) {
-                        V3<double> dr = force_pos<Real, IO>(S, S.bondOther[b]) - pa;
-                        double r = sqrt(dot(dr, dr));
-                        double ext = r - S.bondLen[b];
-                        fd = fd + dr * (S.bondK[b] * ext / r);
-                        if (ENERGY) e[0] += 0.25 * S.bondK[b] * ext * ext;
+        constexpr int U = force_batch<Real, IO>();
+        const bool tethered = S.tetherScale != 0.0;
+        for (int i0 = threadIdx.x; i0 < tile.count; i0 += U * blockDim.x) {
+            int at[U];
+            V3<Real> ph[U], pl[U], r0[U];
+            Real k[U];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (i0 + u * (int)blockDim.x < tile.count) at[u] = IO::at(S, tile.first + i0 + u * blockDim.x);
+            if (tethered) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int a = tile.first + i0 + u * blockDim.x;
+                    if (i0 + u * (int)blockDim.x < tile.count) {
+                        field_pos_parts<Real, IO>(S, a, at[u], ph[u], pl[u]);
+                        r0[u] = ld3<Real>(S.r0, S.atomStride, a);
+                        k[u] = S.tetherUniform ? (Real)S.tetherK0 : reinterpret_cast<const Real*>(S.tetherK)[a];
                     }
-                    f = cvt<Real>(fd);
                 }
             }
-            store_force<Real, IO>(S, a, f);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (i0 + u * (int)blockDim.x >= tile.count) break;
+                const int a = tile.first + i0 + u * blockDim.x;
+                V3<Real> f = {(Real)0, (Real)0, (Real)0};
+                if (tethered) {
+                    V3<Real> dx = (ph[u] - r0[u]) + pl[u];
+                    f = tether_force(dx, k[u]);
+                    if (ENERGY) {
+                        V3<double> dd = cvt<double>(dx);
+                        e[0] += 0.5 * (double)k[u] * dot(dd, dd);
+                    }
+                }
+                if (S.bondStart) {
+                    int e0 = S.bondStart[a], e1 = S.bondStart[a + 1];
+                    if (e0 < e1) {
+                        V3<double> pa = force_pos<Real, IO>(S, a);
+                        V3<double> fd = cvt<double>(f);
+                        for (int b = e0; b < e1; b++) {
+                            V3<double> dr = force_pos<Real, IO>(S, S.bondOther[b]) - pa;
+                            double r = sqrt(dot(dr, dr));
+                            double ext = r - S.bondLen[b];
+                            fd = fd + dr * (S.bondK[b] * ext / r);
+                            if (ENERGY) e[0] += 0.25 * S.bondK[b] * ext * ext;
+                        }
+                        f = cvt<Real>(fd);
+                    }
+                }
+                store_force<Real, IO>(S, at[u], f);
+            }
         }
         if (ENERGY) block_reduce_store<1>(e, S.pePart, tile.slot);
     }
@@ -1542,7 +1625,8 @@ __device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, 
         for (int u = 0; u < per; u++) {
             const V3<Real> d = {st[7 * u], st[7 * u + 1], st[7 * u + 2]};
             const V3<Real> dl = !fixed ? strided_apply(R, d, u) : small ? place_apply<true>(R, d) : step_apply<true>(R, d);
-            IO::template set_body_pos<Real>(S, atom0 + sub + u * lanes, rc + cvt<double>(dl));
+            const int at = IO::at(S, atom0 + sub + u * lanes);
+            IO::template set_body_pos_at<Real>(S, at, rc + cvt<double>(dl));
         }
     }
 }
