@@ -426,7 +426,7 @@ struct rbhip_context {
     int numMassless = 0, numSites = 0, numSiteParents = 0;
     DeviceArena siteArena;
     std::vector<int> clusterN;                   // atoms per cluster (small classes first)
-    std::vector<int> clusterK;                   // constraints per cluster
+    std::vector<int> clusterClass;               // 2, 3 or 4: held in registers, 0: the others
     // built on the device: the reference's cleanBodyIndices result and
     // atomIndex, and the internal order (internal atom -> original atom)
     int* dRefBodyIndex = nullptr;
@@ -691,14 +691,11 @@ struct rbhip_context {
     // registers, or N = 0 for the others), KE slots from slot0
     std::vector<Tile> clusterTiles(int slot0) const {
         std::vector<Tile> t;
-        auto cls = [&](int c) {
-            int n = clusterN[c];
-            return n <= 4 && clusterK[c] <= n * (n - 1) / 2 ? n : 0;
-        };
+        const std::vector<int>& cls = clusterClass;
         for (int c = 0; c < numClusters;) {
             int e = c;
-            while (e < numClusters && e - c < kClusterBlock && cls(e) == cls(c)) e++;
-            Tile x{0, TILE_CLUSTERS, c, e - c, cls(c), 0, 1, slot0 + (int)t.size()};
+            while (e < numClusters && e - c < kClusterBlock && cls[e] == cls[c]) e++;
+            Tile x{0, TILE_CLUSTERS, c, e - c, cls[c], 0, 1, slot0 + (int)t.size()};
             require(x.slot < maxKeSlots, "cluster tile slot out of range", RBHIP_E_STATE);
             t.push_back(x);
             c = e;
@@ -1438,12 +1435,21 @@ static int create_context(int numAtoms, const double* masses, const int* bodyInd
             }
             freeOrder = unconstrained;
             // clusters of n = 2-4 atoms with at most n (n - 1) / 2
-            // constraints first, by size, then the others: each tile holds
-            // one class
-            auto key = [&](int c2) {
-                size_t n = clusterAtoms[c2].size();
-                return n <= 4 && clusterCons[c2].size() <= n * (n - 1) / 2 ? n : 100 + n;
+            // constraints (with 3 atoms: of different pairs) first, by size,
+            // then the others: each tile holds one class
+            auto classOf = [&](int c2) {
+                const size_t n = clusterAtoms[c2].size();
+                const std::vector<int>& cc = clusterCons[c2];
+                if (n > 4 || cc.size() > n * (n - 1) / 2) return 0;
+                if (n == 3 && cc.size() == 3) {
+                    auto sum = [&](int k) { return (long)constraintAtoms[2 * cc[k]] + constraintAtoms[2 * cc[k] + 1]; };
+                    if (sum(0) == sum(1) || sum(1) == sum(2) || sum(0) == sum(2)) return 0;
+                }
+                return (int)n;
             };
+            std::vector<int> classes(clusterAtoms.size());
+            for (size_t c2 = 0; c2 < classes.size(); c2++) classes[c2] = classOf((int)c2);
+            auto key = [&](int c2) { return classes[c2] ? (size_t)classes[c2] : 100 + clusterAtoms[c2].size(); };
             std::vector<int> bySize(clusterAtoms.size());
             for (size_t c2 = 0; c2 < bySize.size(); c2++) bySize[c2] = (int)c2;
             std::stable_sort(bySize.begin(), bySize.end(), [&](int x, int y) { return key(x) < key(y); });
@@ -1454,7 +1460,7 @@ static int create_context(int numAtoms, const double* masses, const int* bodyInd
             }
             clusterAtoms.swap(sortedAtoms);
             clusterCons.swap(sortedCons);
-            for (const auto& cc : clusterCons) C.clusterK.push_back((int)cc.size());
+            for (int c2 : bySize) C.clusterClass.push_back(classes[c2]);
             for (const auto& ca : clusterAtoms) {
                 if ((int)ca.size() > CLUSTER_MAX_ATOMS)
                     throw RbError(RBHIP_E_UNSUPPORTED, "a cluster of constraints joins " + std::to_string(ca.size()) +
