@@ -18,6 +18,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <set>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -427,6 +428,7 @@ struct rbhip_context {
     DeviceArena siteArena;
     std::vector<int> clusterN;                   // atoms per cluster (small classes first)
     std::vector<int> clusterClass;               // 2, 3 or 4: held in registers, 0: the others
+    std::set<int> siteBodySizes;                 // sizes of the bodies that have sites of their own
     // built on the device: the reference's cleanBodyIndices result and
     // atomIndex, and the internal order (internal atom -> original atom)
     int* dRefBodyIndex = nullptr;
@@ -838,13 +840,21 @@ struct rbhip_context {
     }
     // whether launchSteps can carry the system through several steps at once:
     // no atom's force depends on another atom, and a lane's atoms fit its LDS
+    // (a site belongs to its body, a cluster is a whole of its own)
     bool localSteps() const {
-        return !h.bondStart && numSites == 0 && numClusters == 0 &&
-               steps_lds_bytes(precision, atomsPerLane) <= kStepsLdsMax;
+        if (h.bondStart || (numSites > 0 && h.maxBodySites == 0) || clusterClassTiles[3] > 0) return false;
+        for (int n : siteBodySizes) {
+            auto it = lanes.find(n);
+            if (it != lanes.end() && it->second > 1) return false;   // (one lane has the body's atoms)
+        }
+        return steps_lds_bytes(precision, atomsPerLane, h.maxBodySites) <= kStepsLdsMax;
     }
     void launchSteps(int boundaries) {
-        HIPCHK(launch_steps(precision, rotationMode, dSys, dStepTiles, nStepTiles, boundaries, atomsPerLane, stream,
-                            layout()));
+        HIPCHK(launch_steps(precision, rotationMode, dSys, dStepTiles, nStepTiles, boundaries, atomsPerLane,
+                            h.maxBodySites, stream, layout()));
+        if (nClusterTiles > 0)
+            HIPCHK(launch_cluster_steps(precision, dSys, dClusterTiles, clusterClassTiles, boundaries, stream));
+        launchSites();
     }
     int partKeSlots() const { return nPartTiles + nClusterTiles; }
     void launchRefineBegin(bool folded) {
@@ -1213,10 +1223,10 @@ struct rbhip_batch {
     bool localSteps() const {
         for (const rbhip_context* c : members)
             if (c->h.bondStart || c->numSites > 0 || c->numClusters > 0) return false;
-        return steps_lds_bytes(precision, atomsPerLane) <= kStepsLdsMax;
+        return steps_lds_bytes(precision, atomsPerLane, 0) <= kStepsLdsMax;
     }
     void launchSteps(int boundaries) {
-        HIPCHK(launch_steps(precision, rotationMode, dSystems, dStepTiles, nStep, boundaries, atomsPerLane, stream,
+        HIPCHK(launch_steps(precision, rotationMode, dSystems, dStepTiles, nStep, boundaries, atomsPerLane, 0, stream,
                             0));
     }
     void launchRefineBegin(bool folded) {
@@ -1696,10 +1706,44 @@ int rbhip_set_virtual_sites(rbhip_context* ctx, int count, const int* types, con
             }
             ps.push_back((int)pv.size());
         }
+        // each body's sites, if every site is an average of one body's atoms
+        std::vector<int> siteBody(count, -1), bodyStart(C.numBodies + 1, 0), bodySites;
+        std::set<int> sizes;
+        bool own = true;
+        for (int v = 0; v < count && own; v++) {
+            const int np = st[v] == RBHIP_SITE_TWO_AVERAGE ? 2 : 3;
+            own = st[v] == RBHIP_SITE_TWO_AVERAGE || st[v] == RBHIP_SITE_THREE_AVERAGE;
+            for (const auto& cl : C.classes)
+                if (sp[3 * v] >= cl.firstAtom && sp[3 * v] < cl.firstAtom + cl.count * cl.N && cl.N <= kMaxSiteBody) {
+                    siteBody[v] = cl.firstBody + (sp[3 * v] - cl.firstAtom) / cl.N;
+                    const int a0 = cl.firstAtom + (siteBody[v] - cl.firstBody) * cl.N;
+                    for (int k = 0; k < np; k++) own = own && sp[3 * v + k] >= a0 && sp[3 * v + k] < a0 + cl.N;
+                    sizes.insert(cl.N);
+                }
+            own = own && siteBody[v] >= 0;
+        }
+        if (own) {
+            for (int v = 0; v < count; v++) bodyStart[siteBody[v] + 1]++;
+            for (int k = 0; k < C.numBodies; k++) bodyStart[k + 1] += bodyStart[k];
+            bodySites.resize(count);
+            std::vector<int> at(bodyStart.begin(), bodyStart.end() - 1);
+            for (int v = 0; v < count; v++) bodySites[at[siteBody[v]]++] = v;
+        }
         C.setDevice();
         hipStream_t s = C.stream;
         C.siteArena.stream = s;
         DevSys& h = C.h;
+        if (own) {
+            h.bodySiteStart = C.siteArena.allocT<int>(bodyStart.size());
+            h.bodySites = C.siteArena.allocT<int>(bodySites.size());
+            HIPCHK(hipMemcpyAsync(h.bodySiteStart, bodyStart.data(), bodyStart.size() * sizeof(int),
+                                  hipMemcpyHostToDevice, s));
+            HIPCHK(hipMemcpyAsync(h.bodySites, bodySites.data(), bodySites.size() * sizeof(int),
+                                  hipMemcpyHostToDevice, s));
+            for (int k = 0; k < C.numBodies; k++)
+                h.maxBodySites = std::max(h.maxBodySites, bodyStart[k + 1] - bodyStart[k]);
+            C.siteBodySizes = sizes;
+        }
         h.siteAtom = C.siteArena.allocT<int>(sa.size());
         h.siteType = C.siteArena.allocT<int>(st.size());
         h.siteParent = C.siteArena.allocT<int>(sp.size());

@@ -135,6 +135,13 @@ struct DevSys {
     int* parentStart;
     int* parentSite;
     int* parentRole;    // 0, 1, 2: which parent of the site
+    // the sites of each body whose parents all lie in it: bodySites
+    // [bodySiteStart[k], bodySiteStart[k + 1]), at most maxBodySites
+    // (0 unless every site is such a one, a two- or three-particle average)
+    int* bodySiteStart;
+    int* bodySites;
+    int maxBodySites;
+    int pad2;
     // Atom state adopted from a caller in OpenMM's GPU layout (ommSlot ==
     // nullptr: the library's own arrays above hold it).  Per atom slot s:
     //   ommPosq      Real4[s] = (x, y, z, charge)         charge left alone

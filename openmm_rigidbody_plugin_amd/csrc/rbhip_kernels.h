@@ -31,17 +31,26 @@ hipError_t launch_free_ke(int precision, const DevSys* systems, const Tile* tile
 hipError_t launch_fused(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
                         int block, int maxBlocks, hipStream_t stream, int adopted);
 // part 1, then `boundaries` x [forces, fused pass], of systems whose force on
-// an atom depends on that atom alone (no bonds, sites or constraints), each
-// launch carrying its bodies and free atoms through up to kStepsPerLaunch
-// boundaries; the force array is left as it was.  The tiles are those of
-// kStepsBlock-thread workgroups.  atomsPerLane: the most body atoms one lane
-// holds; a launch needs steps_lds_bytes of LDS, at most kStepsLdsMax.
+// an atom depends on that atom alone (no bonds) or, for a virtual site, on its
+// own body (two- and three-particle averages of one body's atoms, held by one
+// lane), each launch carrying its bodies and unconstrained free atoms through
+// up to kStepsPerLaunch boundaries; the force array and the sites are left as
+// they were.  The tiles are those of kStepsBlock-thread workgroups.
+// atomsPerLane: the most body atoms one lane holds; sitesPerLane: the most
+// sites of a body (DevSys::maxBodySites); a launch needs steps_lds_bytes of
+// LDS, at most kStepsLdsMax.
 constexpr int kStepsBlock = 64;
 constexpr int kStepsPerLaunch = 64;
 constexpr size_t kStepsLdsMax = 64 << 10;
-size_t steps_lds_bytes(int precision, int atomsPerLane);
+constexpr int kSiteReals = 14;        // LDS of a site, in state-precision values
+constexpr int kMaxSiteBody = 1000;    // atoms of a body with such sites
+size_t steps_lds_bytes(int precision, int atomsPerLane, int sitesPerLane);
 hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
-                        int boundaries, int atomsPerLane, hipStream_t stream, int adopted);
+                        int boundaries, int atomsPerLane, int sitesPerLane, hipStream_t stream, int adopted);
+// the same for the constraint clusters (tiles and counts as for
+// launch_clusters, no clusters of the last class)
+hipError_t launch_cluster_steps(int precision, const DevSys* systems, const Tile* tiles, const int* counts,
+                                int boundaries, hipStream_t stream);
 // refined energies of the systems whose refBody is set: the start terms of
 // the next step (`folded` = the stored momenta carry its first half-kick,
 // i.e. part1 follows; 0 = a fused boundary follows), the end terms after

@@ -1153,7 +1153,11 @@ template <int NA, int K, class T> __device__ __forceinline__ T second_of(const S
     if constexpr (SmallCons<NA>::kOrdered) return x.template at<kSecond[K]>();
     else return x.template get<NA>(C.cj[K]);
 }
-// v g, rounded (not fused into the sum it goes to)
+// a b and v g, rounded (not fused into the sum they go to)
+__device__ __forceinline__ double product(double a, double b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
 __device__ __forceinline__ V3<double> scaled(V3<double> v, double g) {
 #pragma clang fp contract(off)
     return {v.x * g, v.y * g, v.z * g};
@@ -1180,7 +1184,7 @@ __device__ __forceinline__ bool shake_small(const DevSys& S, const SmallCons<NA>
         static_for<SmallCons<NA>::kMax>([&](auto K) {
             constexpr int k = K;
             if (k >= C.n) return;
-            const double d2 = C.cd[k] * C.cd[k];
+            const double d2 = product(C.cd[k], C.cd[k]);
             V3<double> s = first_of<NA, k>(C, r) - second_of<NA, k>(C, r);
             double s2 = step_dot<true>(s, s);
             if (s2 >= lo * d2 && s2 <= hi * d2) return;
@@ -1218,6 +1222,10 @@ __device__ __forceinline__ bool rattle_small(const DevSys& S, const SmallCons<NA
     return false;
 }
 
+// v + a dt/2, fused
+template <class Real> __device__ __forceinline__ V3<Real> half_kick(V3<Real> v, V3<Real> a, Real halfDt) {
+    return {fma(a.x, halfDt, v.x), fma(a.y, halfDt, v.y), fma(a.z, halfDt, v.z)};
+}
 // a cluster of exactly NA atoms in registers
 template <class Real, int NA> struct SmallCluster {
     Four<int> atom;
@@ -1266,8 +1274,7 @@ template <class Real, int NA> struct SmallCluster {
         Four<V3<double>> vd;
         static_for<NA>([&](auto J) {
             constexpr int j = J;
-            vd.template at<j>() =
-                cvt<double>(v.template at<j>() + f.template at<j>() * invm.template at<j>() * halfDt);
+            vd.template at<j>() = cvt<double>(half_kick(v.template at<j>(), f.template at<j>() * invm.template at<j>(), halfDt));
         });
         const bool ok = rattle_small<NA>(S, C, r, vd, w);
         static_for<NA>([&](auto J) { v.template at<(int)J>() = cvt<Real>(vd.template at<(int)J>()); });
@@ -1279,7 +1286,7 @@ template <class Real, int NA> struct SmallCluster {
         Four<V3<double>> ro, ru;   // before the step, after the drift
         static_for<NA>([&](auto J) {
             constexpr int j = J;
-            v.template at<j>() = v.template at<j>() + f.template at<j>() * invm.template at<j>() * halfDt;
+            v.template at<j>() = half_kick(v.template at<j>(), f.template at<j>() * invm.template at<j>(), halfDt);
             ro.template at<j>() = r.template at<j>();
             r.template at<j>() = r.template at<j>() + cvt<double>(v.template at<j>()) * S.dt;
             ru.template at<j>() = r.template at<j>();
@@ -1585,8 +1592,9 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
 
 // ---------------------------------------------------------------------------
 // Steps of systems whose force on an atom depends on that atom alone (no
-// bonds, sites or constraints: the tether, or no force).  A body's interior
-// step boundaries then need nothing from other bodies, so one launch carries
+// bonds: the tether, or no force), or by way of a virtual site on its own body.
+// A body's interior step boundaries then need nothing from other bodies, and a
+// constraint cluster's nothing from other atoms, so one launch carries
 // each body (each free atom) through `boundaries` x [forces, fused pass] with
 // its state in registers and its atoms' coordinates and anchors in LDS:
 // positions, forces and body state go through memory once per launch instead
@@ -1608,6 +1616,12 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
 // per launch ran the 1M waters at 24.0, 23.4, 23.8 and 23.8 us and the
 // heterogeneous mix at 9.2, 8.6, 8.6 and 8.7; 64 leaves other streams a slot
 // every few ms (a server's set-ups: 29 against 31 ms for a backlog with 2048).
+//
+// Sites and clusters (10k four-site waters and 2000 triangles, per step): six
+// kernels, 31.6 us -> k_steps with the sites 4.1 us and k_cluster_steps 7.0 us,
+// the latter bound by the serial FP64 sweeps of its 32 waves.  A body with
+// sites takes its forces atom by atom in a loop of its own (site_sums), in an
+// instance that systems without sites do not run.
 //
 // LDS: each lane keeps its own atoms' {d, r0, k}, 7 Reals per atom, at an odd
 // stride of Reals, so the lanes of a wave hit different banks; a lane reads
@@ -1655,7 +1669,90 @@ __device__ __forceinline__ void tethered_sums(const Real* st, int N, int per, bo
     }
 }
 
-template <class Real, bool EXACT, class IO>
+// A body's virtual sites, kSiteReals of Real each after its atoms: the weights
+// (FP64), anchor and spring constant, the parents' places in the body, and the
+// force on the site while a step's sums are taken.
+constexpr int kNoParent = 1023;
+template <class Real> struct SiteRecord {
+    Real* a;
+    static constexpr int W = sizeof(double) / sizeof(Real);   // Reals per FP64 value
+    __device__ __forceinline__ void set_weight(int i, double w) { __builtin_memcpy(a + W * i, &w, sizeof(w)); }
+    __device__ __forceinline__ double weight(int i) const {
+        double w;
+        __builtin_memcpy(&w, a + W * i, sizeof(w));
+        return w;
+    }
+    __device__ __forceinline__ V3<Real>& r0() const { return *reinterpret_cast<V3<Real>*>(a + 3 * W); }
+    __device__ __forceinline__ Real& k() const { return a[3 * W + 3]; }
+    __device__ __forceinline__ void set_parents(int p) { __builtin_memcpy(a + 3 * W + 4, &p, sizeof(p)); }
+    __device__ __forceinline__ int parents() const {
+        int p;
+        __builtin_memcpy(&p, a + 3 * W + 4, sizeof(p));
+        return p;
+    }
+    __device__ __forceinline__ V3<Real>& force() const { return *reinterpret_cast<V3<Real>*>(a + 3 * W + 5); }
+};
+
+template <class Real>
+__device__ __forceinline__ void load_site(const DevSys& S, SiteRecord<Real> r, int s, int atom0) {
+    const int a = S.siteAtom[s], two = S.siteType[s] == SITE_TWO_AVERAGE;
+    const int* p = S.siteParent + 3 * (size_t)s;
+    const double* w = S.siteW + 12 * (size_t)s;
+    for (int i = 0; i < 3; i++) r.set_weight(i, w[i]);
+    r.r0() = ld3<Real>(S.r0, S.atomStride, a);
+    r.k() = S.tetherUniform ? (Real)S.tetherK0 : reinterpret_cast<const Real*>(S.tetherK)[a];
+    r.set_parents((p[0] - atom0) | (p[1] - atom0) << 10 | (two ? kNoParent : p[2] - atom0) << 20);
+}
+
+// F and tau of one lane's whole body with sites: as tethered_sums, each force
+// with its share of the sites' forces added and rounded as k_site_forces does
+template <class Real, bool EXACT>
+__device__ __forceinline__ void site_sums(const Real* st, Real* sites, int numSites, int N, bool small, bool uniform,
+                                          Real k0, const Rot<Real>& R, V3<double> rc, V3<double>& F,
+                                          V3<double>& tau) {
+    const bool fixed = N == 2 || N == 3 || N == 4 || N == 6;
+    auto offset = [&](int j) {
+        const V3<Real> d = {st[7 * j], st[7 * j + 1], st[7 * j + 2]};
+        return fixed ? step_apply<true>(R, d) : strided_apply(R, d, j);
+    };
+    auto place = [&](int j) {
+        const V3<Real> d = {st[7 * j], st[7 * j + 1], st[7 * j + 2]};
+        return cvt<Real>(rc + cvt<double>(small ? place_apply<true>(R, d) : offset(j)));
+    };
+    for (int s = 0; s < numSites; s++) {
+        const SiteRecord<Real> r{sites + kSiteReals * s};
+        const int p = r.parents(), p2 = p >> 20 & 1023;
+        const double w0 = r.weight(0), w1 = r.weight(1);
+        const V3<double> x0 = cvt<double>(place(p & 1023)), x1 = cvt<double>(place(p >> 10 & 1023));
+        V3<double> x = {fma(x0.x, w0, x1.x * w1), fma(x0.y, w0, x1.y * w1), fma(x0.z, w0, x1.z * w1)};
+        if (p2 != kNoParent) {
+            const double w2 = r.weight(2);
+            const V3<double> x2 = cvt<double>(place(p2));
+            x = {fma(x2.x, w2, x.x), fma(x2.y, w2, x.y), fma(x2.z, w2, x.z)};
+        }
+        r.force() = tether_force(cvt<Real>(x) - r.r0(), r.k());
+    }
+    for (int j = 0; j < N; j++) {
+        const Real* a = st + 7 * j;
+        V3<double> f = cvt<double>(tether_force(place(j) - V3<Real>{a[3], a[4], a[5]}, uniform ? k0 : a[6]));
+        for (int s = 0; s < numSites; s++) {
+            const SiteRecord<Real> r{sites + kSiteReals * s};
+            const int p = r.parents();
+            const V3<double> fs = cvt<double>(r.force());
+            for (int i = 0; i < 3; i++)
+                if ((p >> 10 * i & 1023) == j) {
+                    const double w = r.weight(i);
+                    f = {fma(fs.x, w, f.x), fma(fs.y, w, f.y), fma(fs.z, w, f.z)};
+                }
+        }
+        f = cvt<double>(cvt<Real>(f));
+        const V3<double> dl = cvt<double>(offset(j));
+        F = F + f;
+        tau = tau + cross(dl, f);
+    }
+}
+
+template <class Real, bool EXACT, class IO, bool SITES>
 __device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, int boundaries, int flags,
                                              Real* stash) {
     const int N = tile.N, lanes = tile.lanes;
@@ -1667,7 +1764,15 @@ __device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, 
     const Shape sh = body_shape(S, tile, k, atom0, N);
     const int perMax = (N + lanes - 1) / lanes;
     const int per = (N - sub + lanes - 1) / lanes;
-    Real* st = stash + (size_t)threadIdx.x * ((7 * perMax) | 1);
+    Real* st = stash + (size_t)threadIdx.x * ((7 * perMax + (SITES ? kSiteReals * S.maxBodySites : 0)) | 1);
+    Real* sites = st + 7 * perMax;
+    int numSites = 0;
+    if constexpr (SITES) {
+        const int first = S.bodySiteStart[k];
+        numSites = S.bodySiteStart[k + 1] - first;
+        for (int s = 0; s < numSites; s++)
+            load_site<Real>(S, SiteRecord<Real>{sites + kSiteReals * s}, S.bodySites[first + s], atom0);
+    }
     const bool tethered = S.tetherScale != 0.0, uniform = S.tetherUniform != 0;
     const Real k0 = (Real)S.tetherK0;
     for (int u = 0; u < per; u++) {
@@ -1687,7 +1792,10 @@ __device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, 
         if (s >= 0) {
             Rot<Real> R = step_rot(B.q);
             V3<double> F = {0.0, 0.0, 0.0}, tau = {0.0, 0.0, 0.0};
-            if (tethered) tethered_sums<Real, EXACT, IO>(st, lanes == 1 ? N : 0, per, uniform, k0, R, rc, F, tau);
+            if (SITES && tethered && numSites > 0)
+                site_sums<Real, EXACT>(st, sites, numSites, N, small, uniform, k0, R, rc, F, tau);
+            else if (tethered)
+                tethered_sums<Real, EXACT, IO>(st, lanes == 1 ? N : 0, per, uniform, k0, R, rc, F, tau);
             if (lanes > 1) {
                 F = {xor_sum(F.x, lanes), xor_sum(F.y, lanes), xor_sum(F.z, lanes)};
                 tau = {xor_sum(tau.x, lanes), xor_sum(tau.y, lanes), xor_sum(tau.z, lanes)};
@@ -1749,7 +1857,7 @@ __device__ __forceinline__ void steps_free(const DevSys& S, const Tile& tile, in
     }
 }
 
-template <class Real, bool EXACT, class IO>
+template <class Real, bool EXACT, class IO, bool SITES>
 __global__ __launch_bounds__(kStepsBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_steps(const DevSys* __restrict__ systems,
                                                               const Tile* __restrict__ tiles, int numTiles,
                                                               int boundaries, int flags) {
@@ -1762,8 +1870,57 @@ __global__ __launch_bounds__(kStepsBlock) __attribute__((amdgpu_waves_per_eu(2))
             steps_free<Real, IO>(S, tile, boundaries, flags);
             continue;
         }
-        steps_bodies<Real, EXACT, IO>(S, tile, boundaries, flags, stash);
+        steps_bodies<Real, EXACT, IO, SITES>(S, tile, boundaries, flags, stash);
     }
+}
+
+// the same for the constraint clusters: a cluster's steps need nothing from
+// other atoms either.  NA = 2, 3 or 4 atoms in registers, one lane each.
+template <class Real, int NA>
+__global__ __launch_bounds__(64) void k_cluster_steps(const DevSys* __restrict__ systems,
+                                                       const Tile* __restrict__ tiles, int boundaries, int flags) {
+    const Tile tile = tiles[blockIdx.x];
+    const DevSys& S = systems[tile.sys];
+    if ((int)threadIdx.x >= tile.count) return;
+    SmallCluster<Real, NA> K;
+    K.load(S, tile.first + threadIdx.x);
+    const bool tethered = S.tetherScale != 0.0;
+    Four<V3<Real>> r0, f;
+    Four<Real> k;
+    static_for<NA>([&](auto J) {
+        constexpr int j = J;
+        const int a = K.atom.template at<j>();
+        r0.template at<j>() = ld3<Real>(S.r0, S.atomStride, a);
+        k.template at<j>() = S.tetherUniform ? (Real)S.tetherK0 : reinterpret_cast<const Real*>(S.tetherK)[a];
+    });
+    // the force at the stored position (hi + lo in mixed precision), to which
+    // the position is rounded
+    auto forces = [&] {
+        static_for<NA>([&](auto J) {
+            constexpr int j = J;
+            V3<double>& r = K.r.template at<j>();
+            V3<Real> hi = cvt<Real>(r), lo = {(Real)0, (Real)0, (Real)0};
+            if (sizeof(Real) == 4) {
+                lo = cvt<Real>(r - cvt<double>(hi));
+                r = cvt<double>(hi) + cvt<double>(lo);
+            }
+            f.template at<j>() = tethered ? tether_force((hi - r0.template at<j>()) + lo, k.template at<j>())
+                                          : V3<Real>{(Real)0, (Real)0, (Real)0};
+        });
+    };
+    unsigned failed = 0;
+    if (flags & STEPS_FIRST) {
+        f = K.stored_forces(S);
+        failed += !K.begin_step(S, f);
+    }
+    for (int s = 0; s < boundaries; s++) {
+        forces();
+        const bool ended = K.end_step(S, f), begun = K.begin_step(S, f);
+        failed += !(ended && begun);
+    }
+    K.store_positions(S);
+    K.store_velocities(S);
+    if (failed) atomicAdd(S.constraintFail, failed);
 }
 
 // deterministic sum of the 4-double partials of each system; one block per
@@ -2051,42 +2208,74 @@ hipError_t launch_forces(int precision, const DevSys* systems, const Tile* tiles
     return hipGetLastError();
 }
 
-template <class IO>
+template <class IO, bool SITES>
 static void steps_for(int precision, int rotationMode, int grid, size_t lds, hipStream_t stream,
                       const DevSys* systems, const Tile* tiles, int numTiles, int boundaries, int flags) {
     auto go = [&](auto kernel) {
         step_kernel_lds(kernel, grid, kStepsBlock, lds, stream, systems, tiles, numTiles, boundaries, flags);
     };
     if (precision == 0) {
-        if (rotationMode == 0) go(k_steps<float, true, IO>);
-        else go(k_steps<float, false, IO>);
+        if (rotationMode == 0) go(k_steps<float, true, IO, SITES>);
+        else go(k_steps<float, false, IO, SITES>);
     } else {
-        if (rotationMode == 0) go(k_steps<double, true, IO>);
-        else go(k_steps<double, false, IO>);
+        if (rotationMode == 0) go(k_steps<double, true, IO, SITES>);
+        else go(k_steps<double, false, IO, SITES>);
     }
 }
 
-size_t steps_lds_bytes(int precision, int atomsPerLane) {
-    return (size_t)kStepsBlock * ((7 * (size_t)atomsPerLane) | 1) * (precision == 0 ? sizeof(float) : sizeof(double));
+size_t steps_lds_bytes(int precision, int atomsPerLane, int sitesPerLane) {
+    const size_t reals = 7 * (size_t)atomsPerLane + (size_t)kSiteReals * sitesPerLane;
+    return (size_t)kStepsBlock * (reals | 1) * (precision == 0 ? sizeof(float) : sizeof(double));
 }
 
-hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
-                        int boundaries, int atomsPerLane, hipStream_t stream, int adopted) {
-    if (numTiles <= 0) return hipSuccess;
-    const size_t lds = steps_lds_bytes(precision, atomsPerLane);
-    if (lds > kStepsLdsMax) return hipErrorInvalidValue;
+// (boundaries, flags) of the launches that carry a system through
+// `boundaries` step boundaries, the last one's with STEPS_LAST
+template <class Launch> static hipError_t steps_launches(int boundaries, Launch&& launch) {
     int flags = STEPS_FIRST;
     do {
         const int n = boundaries < kStepsPerLaunch ? boundaries : kStepsPerLaunch;
         boundaries -= n;
         if (boundaries == 0) flags |= STEPS_LAST;
-        if (adopted) steps_for<AdoptedAtoms>(precision, rotationMode, numTiles, lds, stream, systems, tiles, numTiles, n, flags);
-        else steps_for<SoaAtoms>(precision, rotationMode, numTiles, lds, stream, systems, tiles, numTiles, n, flags);
+        launch(n, flags);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         flags = 0;
     } while (boundaries > 0);
     return hipSuccess;
+}
+
+hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
+                        int boundaries, int atomsPerLane, int sitesPerLane, hipStream_t stream, int adopted) {
+    if (numTiles <= 0) return hipSuccess;
+    const size_t lds = steps_lds_bytes(precision, atomsPerLane, sitesPerLane);
+    if (lds > kStepsLdsMax || (adopted && sitesPerLane)) return hipErrorInvalidValue;
+    return steps_launches(boundaries, [&](int n, int flags) {
+        if (adopted)
+            steps_for<AdoptedAtoms, false>(precision, rotationMode, numTiles, lds, stream, systems, tiles, numTiles, n, flags);
+        else if (sitesPerLane)
+            steps_for<SoaAtoms, true>(precision, rotationMode, numTiles, lds, stream, systems, tiles, numTiles, n, flags);
+        else
+            steps_for<SoaAtoms, false>(precision, rotationMode, numTiles, lds, stream, systems, tiles, numTiles, n, flags);
+    });
+}
+
+template <class Real>
+static void cluster_steps_classes(const DevSys* systems, const Tile* tiles, const int* counts, int boundaries,
+                                  int flags, hipStream_t stream) {
+    if (counts[0]) k_cluster_steps<Real, 2><<<counts[0], 64, 0, stream>>>(systems, tiles, boundaries, flags);
+    tiles += counts[0];
+    if (counts[1]) k_cluster_steps<Real, 3><<<counts[1], 64, 0, stream>>>(systems, tiles, boundaries, flags);
+    tiles += counts[1];
+    if (counts[2]) k_cluster_steps<Real, 4><<<counts[2], 64, 0, stream>>>(systems, tiles, boundaries, flags);
+}
+
+hipError_t launch_cluster_steps(int precision, const DevSys* systems, const Tile* tiles, const int* counts,
+                                int boundaries, hipStream_t stream) {
+    if (counts[3]) return hipErrorInvalidValue;
+    return steps_launches(boundaries, [&](int n, int flags) {
+        if (precision == 0) cluster_steps_classes<float>(systems, tiles, counts, n, flags, stream);
+        else cluster_steps_classes<double>(systems, tiles, counts, n, flags, stream);
+    });
 }
 
 hipError_t launch_reduce(const DevSys* systems, const int* nslots, int numSystems, int which, double* out,
