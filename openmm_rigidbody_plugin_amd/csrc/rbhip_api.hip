@@ -850,10 +850,12 @@ struct rbhip_context {
         return steps_lds_bytes(precision, atomsPerLane, h.maxBodySites) <= kStepsLdsMax;
     }
     void launchSteps(int boundaries) {
-        HIPCHK(launch_steps(precision, rotationMode, dSys, dStepTiles, nStepTiles, boundaries, atomsPerLane,
-                            h.maxBodySites, stream, layout()));
         if (nClusterTiles > 0)
-            HIPCHK(launch_cluster_steps(precision, dSys, dClusterTiles, clusterClassTiles, boundaries, stream));
+            HIPCHK(launch_steps_with_clusters(precision, rotationMode, dSys, dStepTiles, nStepTiles, dClusterTiles,
+                                              clusterClassTiles, boundaries, atomsPerLane, h.maxBodySites, stream));
+        else
+            HIPCHK(launch_steps(precision, rotationMode, dSys, dStepTiles, nStepTiles, boundaries, atomsPerLane,
+                                h.maxBodySites, stream, layout()));
         launchSites();
     }
     int partKeSlots() const { return nPartTiles + nClusterTiles; }

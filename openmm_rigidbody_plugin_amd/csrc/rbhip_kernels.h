@@ -47,10 +47,11 @@ constexpr int kMaxSiteBody = 1000;    // atoms of a body with such sites
 size_t steps_lds_bytes(int precision, int atomsPerLane, int sitesPerLane);
 hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
                         int boundaries, int atomsPerLane, int sitesPerLane, hipStream_t stream, int adopted);
-// the same for the constraint clusters (tiles and counts as for
+// the same with the system's constraint clusters (tiles and counts as for
 // launch_clusters, no clusters of the last class)
-hipError_t launch_cluster_steps(int precision, const DevSys* systems, const Tile* tiles, const int* counts,
-                                int boundaries, hipStream_t stream);
+hipError_t launch_steps_with_clusters(int precision, int rotationMode, const DevSys* systems, const Tile* tiles,
+                                      int numTiles, const Tile* clusterTiles, const int* counts, int boundaries,
+                                      int atomsPerLane, int sitesPerLane, hipStream_t stream);
 // refined energies of the systems whose refBody is set: the start terms of
 // the next step (`folded` = the stored momenta carry its first half-kick,
 // i.e. part1 follows; 0 = a fused boundary follows), the end terms after

@@ -1618,8 +1618,9 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
 // every few ms (a server's set-ups: 29 against 31 ms for a backlog with 2048).
 //
 // Sites and clusters (10k four-site waters and 2000 triangles, per step): six
-// kernels, 31.6 us -> k_steps with the sites 4.1 us and k_cluster_steps 7.0 us,
-// the latter bound by the serial FP64 sweeps of its 32 waves.  A body with
+// kernels, 31.6 us -> bodies and sites 4.1 us beside clusters 7.0 us, the latter
+// bound by the serial FP64 sweeps of their 32 waves (fewer clusters per wave, so
+// that a wave waits for fewer sweeps, were slower: 8.0 with 16, 13.7 with 2).  A body with
 // sites takes its forces atom by atom in a loop of its own (site_sums), in an
 // instance that systems without sites do not run.
 //
@@ -1768,10 +1769,12 @@ __device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, 
     Real* sites = st + 7 * perMax;
     int numSites = 0;
     if constexpr (SITES) {
-        const int first = S.bodySiteStart[k];
-        numSites = S.bodySiteStart[k + 1] - first;
-        for (int s = 0; s < numSites; s++)
-            load_site<Real>(S, SiteRecord<Real>{sites + kSiteReals * s}, S.bodySites[first + s], atom0);
+        if (S.maxBodySites > 0) {
+            const int first = S.bodySiteStart[k];
+            numSites = S.bodySiteStart[k + 1] - first;
+            for (int s = 0; s < numSites; s++)
+                load_site<Real>(S, SiteRecord<Real>{sites + kSiteReals * s}, S.bodySites[first + s], atom0);
+        }
     }
     const bool tethered = S.tetherScale != 0.0, uniform = S.tetherUniform != 0;
     const Real k0 = (Real)S.tetherK0;
@@ -1857,33 +1860,11 @@ __device__ __forceinline__ void steps_free(const DevSys& S, const Tile& tile, in
     }
 }
 
-template <class Real, bool EXACT, class IO, bool SITES>
-__global__ __launch_bounds__(kStepsBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_steps(const DevSys* __restrict__ systems,
-                                                              const Tile* __restrict__ tiles, int numTiles,
-                                                              int boundaries, int flags) {
-    extern __shared__ double stash_memory[];
-    Real* stash = reinterpret_cast<Real*>(stash_memory);
-    for (int t = blockIdx.x; t < numTiles; t += gridDim.x) {
-        const Tile tile = tiles[t];
-        const DevSys& S = systems[tile.sys];
-        if (tile.kind == TILE_FREE) {
-            steps_free<Real, IO>(S, tile, boundaries, flags);
-            continue;
-        }
-        steps_bodies<Real, EXACT, IO, SITES>(S, tile, boundaries, flags, stash);
-    }
-}
-
-// the same for the constraint clusters: a cluster's steps need nothing from
-// other atoms either.  NA = 2, 3 or 4 atoms in registers, one lane each.
+// the same for one constraint cluster of NA atoms
 template <class Real, int NA>
-__global__ __launch_bounds__(64) void k_cluster_steps(const DevSys* __restrict__ systems,
-                                                       const Tile* __restrict__ tiles, int boundaries, int flags) {
-    const Tile tile = tiles[blockIdx.x];
-    const DevSys& S = systems[tile.sys];
-    if ((int)threadIdx.x >= tile.count) return;
+__device__ __forceinline__ void steps_cluster(const DevSys& S, int c, int boundaries, int flags) {
     SmallCluster<Real, NA> K;
-    K.load(S, tile.first + threadIdx.x);
+    K.load(S, c);
     const bool tethered = S.tetherScale != 0.0;
     Four<V3<Real>> r0, f;
     Four<Real> k;
@@ -1921,6 +1902,54 @@ __global__ __launch_bounds__(64) void k_cluster_steps(const DevSys* __restrict__
     K.store_positions(S);
     K.store_velocities(S);
     if (failed) atomicAdd(S.constraintFail, failed);
+}
+
+template <class Real, bool EXACT, class IO, bool SITES>
+__global__ __launch_bounds__(kStepsBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_steps(const DevSys* __restrict__ systems,
+                                                              const Tile* __restrict__ tiles, int numTiles,
+                                                              int boundaries, int flags) {
+    extern __shared__ double stash_memory[];
+    Real* stash = reinterpret_cast<Real*>(stash_memory);
+    for (int t = blockIdx.x; t < numTiles; t += gridDim.x) {
+        const Tile tile = tiles[t];
+        const DevSys& S = systems[tile.sys];
+        if (tile.kind == TILE_FREE) {
+            steps_free<Real, IO>(S, tile, boundaries, flags);
+            continue;
+        }
+        steps_bodies<Real, EXACT, IO, SITES>(S, tile, boundaries, flags, stash);
+    }
+}
+
+// constraint clusters of NA = 2, 3 or 4 atoms, one lane each
+template <class Real, int NA>
+__global__ __launch_bounds__(kStepsBlock) void k_cluster_steps(const DevSys* __restrict__ systems,
+                                                               const Tile* __restrict__ tiles, int boundaries,
+                                                               int flags) {
+    const Tile tile = tiles[blockIdx.x];
+    const DevSys& S = systems[tile.sys];
+    if ((int)threadIdx.x < tile.count) steps_cluster<Real, NA>(S, tile.first + threadIdx.x, boundaries, flags);
+}
+
+// bodies, free atoms and clusters of 2 and 3 atoms side by side, the clusters,
+// which take longest, first
+template <class Real, bool EXACT>
+__global__ __launch_bounds__(kStepsBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_steps_mixed(
+    const DevSys* __restrict__ systems, const Tile* __restrict__ tiles, const Tile* __restrict__ clusterTiles,
+    int numClusterTiles, int boundaries, int flags) {
+    extern __shared__ double stash_memory[];
+    const int t = (int)blockIdx.x - numClusterTiles;
+    const Tile tile = t < 0 ? clusterTiles[blockIdx.x] : tiles[t];
+    const DevSys& S = systems[tile.sys];
+    if (tile.kind == TILE_CLUSTERS) {
+        if ((int)threadIdx.x >= tile.count) return;
+        if (tile.N == 2) steps_cluster<Real, 2>(S, tile.first + threadIdx.x, boundaries, flags);
+        else steps_cluster<Real, 3>(S, tile.first + threadIdx.x, boundaries, flags);
+    } else if (tile.kind == TILE_FREE) {
+        steps_free<Real, SoaAtoms>(S, tile, boundaries, flags);
+    } else {
+        steps_bodies<Real, EXACT, SoaAtoms, true>(S, tile, boundaries, flags, reinterpret_cast<Real*>(stash_memory));
+    }
 }
 
 // deterministic sum of the 4-double partials of each system; one block per
@@ -2262,19 +2291,51 @@ hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, 
 template <class Real>
 static void cluster_steps_classes(const DevSys* systems, const Tile* tiles, const int* counts, int boundaries,
                                   int flags, hipStream_t stream) {
-    if (counts[0]) k_cluster_steps<Real, 2><<<counts[0], 64, 0, stream>>>(systems, tiles, boundaries, flags);
-    tiles += counts[0];
-    if (counts[1]) k_cluster_steps<Real, 3><<<counts[1], 64, 0, stream>>>(systems, tiles, boundaries, flags);
-    tiles += counts[1];
-    if (counts[2]) k_cluster_steps<Real, 4><<<counts[2], 64, 0, stream>>>(systems, tiles, boundaries, flags);
+    auto go = [&](auto kernel, int n) {
+        if (n) kernel<<<n, kStepsBlock, 0, stream>>>(systems, tiles, boundaries, flags);
+        tiles += n;
+    };
+    go(k_cluster_steps<Real, 2>, counts[0]);
+    go(k_cluster_steps<Real, 3>, counts[1]);
+    go(k_cluster_steps<Real, 4>, counts[2]);
 }
 
-hipError_t launch_cluster_steps(int precision, const DevSys* systems, const Tile* tiles, const int* counts,
-                                int boundaries, hipStream_t stream) {
-    if (counts[3]) return hipErrorInvalidValue;
+// One launch for both takes as long as the longer, where two take the sum
+// (10k four-site waters and 2000 triangles, 49 boundaries: 203 + 342 us, 345
+// together).  Its registers allow 2 waves per SIMD, where the bodies alone run
+// 4: so while all of its workgroups are resident at once on 1024 SIMDs.
+// Clusters of 4 atoms need more registers than that.
+static bool steps_together(int numTiles, const int* counts) {
+    return counts[2] == 0 && numTiles + counts[0] + counts[1] <= 2048;
+}
+
+hipError_t launch_steps_with_clusters(int precision, int rotationMode, const DevSys* systems, const Tile* tiles,
+                                      int numTiles, const Tile* clusterTiles, const int* counts, int boundaries,
+                                      int atomsPerLane, int sitesPerLane, hipStream_t stream) {
+    const size_t lds = steps_lds_bytes(precision, atomsPerLane, sitesPerLane);
+    if (lds > kStepsLdsMax || counts[3]) return hipErrorInvalidValue;
+    if (steps_together(numTiles, counts)) {
+        const int nc = counts[0] + counts[1];
+        return steps_launches(boundaries, [&](int n, int flags) {
+            auto go = [&](auto kernel) {
+                step_kernel_lds(kernel, nc + numTiles, kStepsBlock, lds, stream, systems, tiles, clusterTiles, nc, n,
+                                flags);
+            };
+            if (precision == 0) {
+                if (rotationMode == 0) go(k_steps_mixed<float, true>);
+                else go(k_steps_mixed<float, false>);
+            } else {
+                if (rotationMode == 0) go(k_steps_mixed<double, true>);
+                else go(k_steps_mixed<double, false>);
+            }
+        });
+    }
+    hipError_t e = launch_steps(precision, rotationMode, systems, tiles, numTiles, boundaries, atomsPerLane,
+                                sitesPerLane, stream, 0);
+    if (e != hipSuccess) return e;
     return steps_launches(boundaries, [&](int n, int flags) {
-        if (precision == 0) cluster_steps_classes<float>(systems, tiles, counts, n, flags, stream);
-        else cluster_steps_classes<double>(systems, tiles, counts, n, flags, stream);
+        if (precision == 0) cluster_steps_classes<float>(systems, clusterTiles, counts, n, flags, stream);
+        else cluster_steps_classes<double>(systems, clusterTiles, counts, n, flags, stream);
     });
 }
 
