@@ -6,9 +6,10 @@ Workload (default): 1,000,000 water-like 3-site rigid bodies (3M atoms) on a
 jittered 100^3 lattice in a 21.5 nm box, 300 K velocities, harmonic tethers
 k = 1000 kJ/mol/nm^2, dt = 2 fs, NO-SQUISH n = 10, mixed precision (fp32
 state, FP64 accumulation); synthetic seeded data.  The timed region is one
-RigidBodyIntegrator::step(K) call: part1, forces, (K-1) x [fused part2+part1,
-forces], part2 -- one step per body per fused pass plus one tether force
-evaluation per step.
+RigidBodyIntegrator::step(K) call: part1, forces, (K-1) x [part2+part1, forces],
+part2 -- every body takes every step with its tether forces evaluated at every
+step, up to 64 of them per launch.  The step kernels that run one step at a
+time (part1, forces, part2, fused) are timed beside it.
 
 Prints one JSON line: whole-job body-steps/s over K timed steps (inputs
 resident in HBM), the HBM roofline of the dominant integrator kernel measured
@@ -213,8 +214,8 @@ def plain_run(ctxs, steps, per_step):
     """Steps each context in turn through its own calls.  per_step: the
     reference's execute pattern (part1, forces, part2 launched for every
     step, as an OpenMM integration does with OpenMM computing the forces);
-    otherwise one step(K) call per context (fused boundaries, HIP-graph
-    replay).  Returns the seconds taken."""
+    otherwise one step(K) call per context (several steps per launch).
+    Returns the seconds taken."""
     from openmm_rigidbody_plugin_amd import rbhip
     for c in ctxs:
         c.use_fusion(not per_step)
@@ -236,8 +237,8 @@ def batched(steps, warmup, count=256, log_every=64, plain=True):
     / 20% argon, k ~ U[500, 2000]) stepped `steps` times: one system at a time
     (each context on its own stream) with per-step launches and with step(K)
     (unless `plain` is false), then all of them as one batch (one launch per
-    phase over every replica's tiles, HIP-graph replay, launch shape from the
-    batch autotuner), and the batch's kernels timed on their own dispatches."""
+    phase or per several steps over every replica's tiles, launch shape from
+    the batch autotuner), and the batch's kernels timed on their own dispatches."""
     from openmm_rigidbody_plugin_amd import rbhip, systems
     t = time.perf_counter()
     specs = systems.replica_set(count)
@@ -454,8 +455,9 @@ def kernel_roofline(kms, natoms_body, nb, nf, config, shared_frames=False):
             "valu_issue_frac_recorded": valu_from_profiles(config, dominant),
         },
         "integrator": {
-            "note": "step(K) runs one fused pass and one force evaluation per step; the two-pass step "
-                    "(part1 + part2, one execute() with the forces computed outside the library) beside it",
+            "note": "the kernels that take one step at a time: the fused pass (interior steps of systems with "
+                    "bonds; this workload's run several to a launch), and the two-pass step (part1 + part2, "
+                    "one execute() with the forces computed outside the library) beside it",
             "fused_ms_per_step": kms["fused"],
             "fused_body_steps_per_s": nb / (kms["fused"] * 1e-3),
             "two_pass_ms_per_step": two_ms,
