@@ -287,10 +287,11 @@ int rbhip_part2(rbhip_context* ctx);
    trajectory as steps x [part1, forces, part2] (bit for bit in mixed
    precision, to a few ulp in FP64), without the interior steps' atom
    velocities and kinetic energies, which nothing reads.
-   Where no atom's force depends on another atom (the tether alone), the
-   interior boundaries run up to 64 per launch with the state in registers.
-   Long sequences of steps with clusters or sites are replayed from a HIP
-   graph when enabled. */
+   Without bonds, and with every virtual site a two- or three-particle average
+   of one body's atoms and every cluster of constraints of at most 4 atoms,
+   the interior boundaries run up to 64 per launch with the state in
+   registers.  Long sequences of steps with other sites or clusters are
+   replayed from a HIP graph when enabled. */
 int rbhip_execute(rbhip_context* ctx, int steps);
 /* 1 = capture the repeated launches of long sequences in a HIP graph and
    replay it where that is faster (default) */
