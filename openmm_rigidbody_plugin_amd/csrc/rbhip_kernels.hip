@@ -1484,7 +1484,7 @@ __global__ __launch_bounds__(256) void k_site_forces(const DevSys* __restrict__ 
         V3<double> fs = cvt<double>(ld3<Real>(S.force, S.atomStride, S.siteAtom[s]));
         const int type = S.siteType[s];
         if (type == SITE_TWO_AVERAGE || type == SITE_THREE_AVERAGE) {
-            f = f + fs * w[role];
+            f = f + scaled(fs, w[role]);
         } else if (type == SITE_LOCAL_COORDINATES) {
             // ow F + xw Gx + yw Gy, Gx and Gy the transposed derivatives of
             // the site with respect to x and y
@@ -1749,10 +1749,7 @@ __device__ __forceinline__ void site_sums(const Real* st, Real* sites, int numSi
             const int p = r.parents();
             const V3<double> fs = cvt<double>(r.force());
             for (int i = 0; i < 3; i++)
-                if ((p >> 10 * i & 1023) == j) {
-                    const double w = r.weight(i);
-                    f = {fma(fs.x, w, f.x), fma(fs.y, w, f.y), fma(fs.z, w, f.z)};
-                }
+                if ((p >> 10 * i & 1023) == j) f = f + scaled(fs, r.weight(i));
         }
         f = cvt<double>(cvt<Real>(f));
         const V3<double> dl = cvt<double>(offset(j));
