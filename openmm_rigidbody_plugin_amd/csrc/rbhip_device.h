@@ -105,6 +105,15 @@ template <bool YFIRST, class T> __device__ __forceinline__ T step_dot(V3<T> u, V
 template <bool YFIRST, class T> __device__ __forceinline__ V3<T> step_apply(const Rot<T>& R, V3<T> x) {
     return {step_dot<YFIRST>(R.r0, x), step_dot<YFIRST>(R.r1, x), step_dot<YFIRST>(R.r2, x)};
 }
+// a b and v g, rounded (not fused into the sum they go to)
+__device__ __forceinline__ double product(double a, double b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+__device__ __forceinline__ V3<double> scaled(V3<double> v, double g) {
+#pragma clang fp contract(off)
+    return {v.x * g, v.y * g, v.z * g};
+}
 // for an atom's position: SMALL (bodies of 2 to 4 atoms on one lane under
 // NO-SQUISH) rounds the x product of the first row
 template <bool SMALL, class T> __device__ __forceinline__ V3<T> place_apply(const Rot<T>& R, V3<T> x) {

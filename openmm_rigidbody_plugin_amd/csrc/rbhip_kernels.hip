@@ -289,8 +289,9 @@ __device__ __forceinline__ void body_velocities(const DevSys& S, const Rot<Real>
     }
 }
 // A(q) x from the rows of A(q)^T, fused operations written out as in
-// step_apply: the y product rounded, or the x product for the bodies whose
-// NO-SQUISH fused pass keeps them in registers (one lane, 2 to 4 atoms)
+// step_apply: the y product rounded, or, in the fused pass, the x product for
+// the bodies that its NO-SQUISH form keeps in registers (one lane, 2 to 4
+// atoms; an FP64 unit in the last place of a torque's moment)
 template <class Real> __device__ __forceinline__ V3<double> to_body(const Rot<Real>& R, V3<double> x, bool small) {
     const V3<double> r0 = cvt<double>(R.r0), r1 = cvt<double>(R.r1), r2 = cvt<double>(R.r2);
     if (small)
@@ -299,8 +300,7 @@ template <class Real> __device__ __forceinline__ V3<double> to_body(const Rot<Re
     return {fma(r2.x, x.z, fma(r0.x, x.x, r1.x * x.y)), fma(r2.y, x.z, fma(r0.y, x.x, r1.y * x.y)),
             fma(r2.z, x.z, fma(r0.z, x.x, r1.z * x.y))};
 }
-// p + F h, fused (in part 2 the product is used twice, which would otherwise
-// be rounded there and not in the fused pass)
+// p + F h, fused
 __device__ __forceinline__ V3<double> kicked(V3<double> p, V3<double> F, double h) {
     return {fma(F.x, h, p.x), fma(F.y, h, p.y), fma(F.z, h, p.z)};
 }
@@ -517,7 +517,7 @@ __device__ __forceinline__ void part2_bodies(const DevSys& S, const Tile& tile, 
     body_sums_any<Real, IO>(S, R, atom0, dbase, N, sub, tile.lanes, active, F, tau);
     if (!active) return;
     const double halfDt = 0.5 * S.dt;
-    V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
+    V3<double> tb = axial_torque(to_body(R, tau, false), B.invI);
     V3<double> p = kicked(cvt<double>(B.p), F, halfDt);
     V3<double> L = kicked(cvt<double>(B.L), tb, halfDt);
     V3<double> w = hadamard(cvt<double>(B.invI), L);
@@ -533,9 +533,10 @@ __device__ __forceinline__ void part2_bodies(const DevSys& S, const Tile& tile, 
     if (sub == 0) {
         ke[0] = dot(p, vcm);
         ke[1] = dot(L, w);
-        // first half-kick of the next step (same F and torque)
-        stp3<Real>(S.pcm, k, cvt<Real>(kicked(p, F, halfDt)));
-        stp3<Real>(S.L, k, cvt<Real>(kicked(L, tb, halfDt)));
+        // first half-kick of the next step (same F and torque), its product
+        // rounded before it is added
+        stp3<Real>(S.pcm, k, cvt<Real>(p + scaled(F, halfDt)));
+        stp3<Real>(S.L, k, cvt<Real>(L + scaled(tb, halfDt)));
     }
 }
 
@@ -745,7 +746,7 @@ __device__ __forceinline__ void refine_begin_bodies(const DevSys& S, const Tile&
     V3<double> F, tau;
     body_sums_any<Real, IO>(S, R, atom0, sh.row, tile.N, sub, tile.lanes, active, F, tau);
     if (!active || sub != 0) return;
-    V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
+    V3<double> tb = axial_torque(to_body(R, tau, false), B.invI);
     V3<double> ar;
     V3<Real> Lback;
     Body<Real> B1 = B;
@@ -755,7 +756,7 @@ __device__ __forceinline__ void refine_begin_bodies(const DevSys& S, const Tile&
         Lback = cvt<Real>(cvt<double>(B.L) + tb * -S.dt);
     } else {
         // stored p = p(t-dt/2), L = L(t) - tau dt/2 (after the last rotation)
-        fused_kicks<Real>(S, B1, R, F, tau, small_body(S, tile.N, tile.lanes));
+        fused_kicks<Real>(S, B1, R, F, tau, false);
         ar = cvt<double>(B1.p) * 5.0 + cvt<double>(B.p) * -1.0;
         Lback = B.L;
     }
@@ -812,7 +813,7 @@ __device__ __forceinline__ void refine_end_bodies(const DevSys& S, const Tile& t
     body_sums_any<Real, IO>(S, R, atom0, sh.row, tile.N, sub, tile.lanes, active, F, tau);
     if (!active || sub != 0) return;
     const double halfDt = 0.5 * S.dt;
-    V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
+    V3<double> tb = axial_torque(to_body(R, tau, false), B.invI);
     V3<double> p1 = cvt<double>(B.p) + F * -halfDt;
     V3<double> L1 = cvt<double>(B.L) + tb * -halfDt;
     Q4<Real> r0 = ld4<Real>(S.refBody, 2 * k), r1 = ld4<Real>(S.refBody, 2 * k + 1);
@@ -874,7 +875,7 @@ __global__ __launch_bounds__(512) void k_refine_pe(const DevSys* __restrict__ sy
             V3<double> F, tau;
             body_sums_any<Real, IO>(S, R, atom0, sh.row, tile.N, sub, tile.lanes, active, F, tau);
             if (active && sub == 0) {
-                V3<double> tb = axial_torque(to_body(R, tau, small_body(S, tile.N, tile.lanes)), B.invI);
+                V3<double> tb = axial_torque(to_body(R, tau, false), B.invI);
                 u[0] = dot(F, F) * (double)B.invM + dot(hadamard(tb, cvt<double>(B.invI)), tb);
             }
         }
@@ -1160,15 +1161,6 @@ template <int NA, int K, class T> __device__ __forceinline__ T first_of(const Sm
 template <int NA, int K, class T> __device__ __forceinline__ T second_of(const SmallCons<NA>& C, Four<T>& x) {
     if constexpr (SmallCons<NA>::kOrdered) return x.template at<kSecond[K]>();
     else return x.template get<NA>(C.cj[K]);
-}
-// a b and v g, rounded (not fused into the sum they go to)
-__device__ __forceinline__ double product(double a, double b) {
-#pragma clang fp contract(off)
-    return a * b;
-}
-__device__ __forceinline__ V3<double> scaled(V3<double> v, double g) {
-#pragma clang fp contract(off)
-    return {v.x * g, v.y * g, v.z * g};
 }
 // x_i += a, x_j += b for the atoms i and j of constraint K
 template <int NA, int K>

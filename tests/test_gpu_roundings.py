@@ -1,0 +1,32 @@
+"""Trajectories pinned to the last bit.  Part 1, part 2, the fused pass and the
+steps kept in registers share one arithmetic whose fused operations are written
+out; what they gave before several steps went through one launch is recorded in
+golden/roundings.npz, and a product that is fused where it was rounded, or the
+other way round, moves it.
+
+Mixed precision: bodies picked from 2e10 body-steps because one FP64 unit in
+the last place decides an fp32 rounding in their trajectory (the exact
+rotation's sums; the placement of 3-atom bodies in the first boundary after a
+part 1).  Double precision: small mixtures, where every such unit shows."""
+import os
+
+import numpy as np
+import pytest
+
+from openmm_rigidbody_plugin_amd import systems
+
+pytestmark = pytest.mark.gpu
+GOLDEN = np.load(os.path.join(os.path.dirname(__file__), "golden", "roundings.npz"))
+CASES = (5, 6)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_recorded_trajectory(hip, case):
+    g = {k.split("_", 1)[1]: GOLDEN[k] for k in GOLDEN.files if k.startswith(f"{case}_")}
+    spec = systems.SystemSpec(masses=g["masses"], body_indices=g["labels"], positions=g["x"], velocities=g["v"],
+                              tether_k=g["k"], tether_r0=g["r0"], dt=float(g["dt"]), rotation_mode=int(g["mode"]))
+    c = hip.Context.from_spec(spec, precision="double" if g["double"] else "mixed")
+    for _ in range(int(g["count"])):
+        c.step(int(g["chunk"]))
+    np.testing.assert_array_equal(c.positions(), g["positions"])
+    np.testing.assert_array_equal(c.velocities(), g["velocities"])
