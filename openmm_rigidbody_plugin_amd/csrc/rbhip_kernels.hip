@@ -1601,7 +1601,8 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
 // of once per step.  The arithmetic and every rounding to the state precision
 // are those of k_part1, k_forces and k_fused (the fused operations whose
 // choice the compiler makes by context are written out: step_rot, step_apply,
-// to_body, kicked), so results are the same bit for bit.
+// to_body, kicked), so results are the same bit for bit as part 1, then
+// [forces, fused pass], gives.
 // FIRST: a part 1 comes before the boundaries; LAST: the atom positions are
 // written at the end (a launch that continues another reads only the body
 // state).
@@ -1635,10 +1636,10 @@ enum : int { STEPS_FIRST = 1, STEPS_LAST = 2 };
 // adds one tethered atom's force and torque to F and tau (a: its {d, r0, k})
 template <class Real, bool YFIRST, bool SMALL, class IO>
 __device__ __forceinline__ void add_tethered(const Real* a, bool uniform, Real k0, const Rot<Real>& R, V3<double> rc,
-                                             V3<double>& F, V3<double>& tau) {
+                                             bool xfirst, V3<double>& F, V3<double>& tau) {
     const V3<Real> d = {a[0], a[1], a[2]};
     V3<double> dl = cvt<double>(step_apply<YFIRST>(R, d));
-    V3<Real> x = cvt<Real>(rc + (SMALL ? cvt<double>(place_apply<true>(R, d)) : dl));
+    V3<Real> x = cvt<Real>(rc + (SMALL && xfirst ? cvt<double>(place_apply<true>(R, d)) : dl));
     V3<double> f = cvt<double>(IO::held_force(tether_force(x - V3<Real>{a[3], a[4], a[5]}, uniform ? k0 : a[6])));
     F = F + f;
     tau = tau + cross(dl, f);
@@ -1649,11 +1650,13 @@ __device__ __forceinline__ void add_tethered(const Real* a, bool uniform, Real k
 // has them all)
 template <class Real, bool EXACT, class IO>
 __device__ __forceinline__ void tethered_sums(const Real* st, int N, int per, bool uniform, Real k0,
-                                              const Rot<Real>& R, V3<double> rc, V3<double>& F, V3<double>& tau) {
+                                              const Rot<Real>& R, V3<double> rc, bool xfirst, V3<double>& F,
+                                              V3<double>& tau) {
     auto fixed = [&](auto NC) {
 #pragma unroll
         for (int u = 0; u < NC; u++)
-            add_tethered<Real, true, (!EXACT && decltype(NC)::value <= 4), IO>(st + 7 * u, uniform, k0, R, rc, F, tau);
+            add_tethered<Real, true, (!EXACT && decltype(NC)::value <= 4), IO>(st + 7 * u, uniform, k0, R, rc, xfirst,
+                                                                               F, tau);
     };
     switch (N) {
     case 2: fixed(std::integral_constant<int, 2>{}); break;
@@ -1662,10 +1665,10 @@ __device__ __forceinline__ void tethered_sums(const Real* st, int N, int per, bo
     case 6: fixed(std::integral_constant<int, 6>{}); break;
     default:
         for (int u0 = 0; u0 < per; u0 += STRIDED_BATCH) {
-            add_tethered<Real, true, false, IO>(st + 7 * u0, uniform, k0, R, rc, F, tau);
+            add_tethered<Real, true, false, IO>(st + 7 * u0, uniform, k0, R, rc, false, F, tau);
             const int end = per < u0 + STRIDED_BATCH ? per : u0 + STRIDED_BATCH;
             for (int u = u0 + 1; u < end; u++)
-                add_tethered<Real, false, false, IO>(st + 7 * u, uniform, k0, R, rc, F, tau);
+                add_tethered<Real, false, false, IO>(st + 7 * u, uniform, k0, R, rc, false, F, tau);
         }
     }
 }
@@ -1708,7 +1711,7 @@ __device__ __forceinline__ void load_site(const DevSys& S, SiteRecord<Real> r, i
 // F and tau of one lane's whole body with sites: as tethered_sums, each force
 // with its share of the sites' forces added and rounded as k_site_forces does
 template <class Real, bool EXACT>
-__device__ __forceinline__ void site_sums(const Real* st, Real* sites, int numSites, int N, bool small, bool uniform,
+__device__ __forceinline__ void site_sums(const Real* st, Real* sites, int numSites, int N, bool xfirst, bool uniform,
                                           Real k0, const Rot<Real>& R, V3<double> rc, V3<double>& F,
                                           V3<double>& tau) {
     const bool fixed = N == 2 || N == 3 || N == 4 || N == 6;
@@ -1718,7 +1721,7 @@ __device__ __forceinline__ void site_sums(const Real* st, Real* sites, int numSi
     };
     auto place = [&](int j) {
         const V3<Real> d = {st[7 * j], st[7 * j + 1], st[7 * j + 2]};
-        return cvt<Real>(rc + cvt<double>(small ? place_apply<true>(R, d) : offset(j)));
+        return cvt<Real>(rc + cvt<double>(xfirst ? place_apply<true>(R, d) : offset(j)));
     };
     for (int s = 0; s < numSites; s++) {
         const SiteRecord<Real> r{sites + kSiteReals * s};
@@ -1788,14 +1791,18 @@ __device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, 
     V3<double> rc = load_rcm<Real>(S, k);
     const bool small = small_body(S, N, lanes);
     const int first = (flags & STEPS_FIRST) ? -1 : 0;
+    // whether step s's positions have row 0's x products rounded: those of
+    // small bodies, where the fused pass places them, and of 4 atoms where
+    // part 1 does (before step 0), which places 2 and 3 the other way
+    auto xfirst = [&](int s) { return small && (N == 4 || s > 0 || !(flags & STEPS_FIRST)); };
     for (int s = first; s < boundaries; s++) {
         if (s >= 0) {
             Rot<Real> R = step_rot(B.q);
             V3<double> F = {0.0, 0.0, 0.0}, tau = {0.0, 0.0, 0.0};
             if (SITES && tethered && numSites > 0)
-                site_sums<Real, EXACT>(st, sites, numSites, N, small, uniform, k0, R, rc, F, tau);
+                site_sums<Real, EXACT>(st, sites, numSites, N, xfirst(s), uniform, k0, R, rc, F, tau);
             else if (tethered)
-                tethered_sums<Real, EXACT, IO>(st, lanes == 1 ? N : 0, per, uniform, k0, R, rc, F, tau);
+                tethered_sums<Real, EXACT, IO>(st, lanes == 1 ? N : 0, per, uniform, k0, R, rc, xfirst(s), F, tau);
             if (lanes > 1) {
                 F = {xor_sum(F.x, lanes), xor_sum(F.y, lanes), xor_sum(F.z, lanes)};
                 tau = {xor_sum(tau.x, lanes), xor_sum(tau.y, lanes), xor_sum(tau.z, lanes)};
@@ -1810,7 +1817,9 @@ __device__ __forceinline__ void steps_bodies(const DevSys& S, const Tile& tile, 
         const bool fixed = lanes == 1 && (N == 2 || N == 3 || N == 4 || N == 6);
         for (int u = 0; u < per; u++) {
             const V3<Real> d = {st[7 * u], st[7 * u + 1], st[7 * u + 2]};
-            const V3<Real> dl = !fixed ? strided_apply(R, d, u) : small ? place_apply<true>(R, d) : step_apply<true>(R, d);
+            const V3<Real> dl = !fixed                ? strided_apply(R, d, u)
+                                : xfirst(boundaries) ? place_apply<true>(R, d)
+                                                     : step_apply<true>(R, d);
             const int at = IO::at(S, atom0 + sub + u * lanes);
             IO::template set_body_pos_at<Real>(S, at, rc + cvt<double>(dl));
         }

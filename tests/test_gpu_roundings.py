@@ -17,7 +17,7 @@ from openmm_rigidbody_plugin_amd import systems
 
 pytestmark = pytest.mark.gpu
 GOLDEN = np.load(os.path.join(os.path.dirname(__file__), "golden", "roundings.npz"))
-CASES = (5, 6)
+CASES = (1, 2, 5, 6, 7)
 
 
 @pytest.mark.parametrize("case", CASES)
