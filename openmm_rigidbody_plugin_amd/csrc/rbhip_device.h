@@ -162,10 +162,17 @@ __device__ __forceinline__ void sin_cosm1_small(float phi, float& s, float& cm1)
     s = phi * fmaf(x2, fmaf(x2, 1.0f / 120.0f, -1.0f / 6.0f), 1.0f);
     cm1 = x2 * fmaf(x2, fmaf(x2, -1.0f / 720.0f, 1.0f / 24.0f), -0.5f);
 }
+// sin(phi) / phi and (cos(phi) - 1) / phi^2 from x2 = phi^2
+__device__ __forceinline__ double sin_series(double x2) {
+    return fma(x2, fma(x2, fma(x2, fma(x2, 1.0 / 362880.0, -1.0 / 5040.0), 1.0 / 120.0), -1.0 / 6.0), 1.0);
+}
+__device__ __forceinline__ double cosm1_series(double x2) {
+    return fma(x2, fma(x2, fma(x2, fma(x2, -1.0 / 3628800.0, 1.0 / 40320.0), -1.0 / 720.0), 1.0 / 24.0), -0.5);
+}
 __device__ __forceinline__ void sin_cosm1_small(double phi, double& s, double& cm1) {
     double x2 = phi * phi;
-    s = phi * fma(x2, fma(x2, fma(x2, fma(x2, 1.0 / 362880.0, -1.0 / 5040.0), 1.0 / 120.0), -1.0 / 6.0), 1.0);
-    cm1 = x2 * fma(x2, fma(x2, fma(x2, fma(x2, -1.0 / 3628800.0, 1.0 / 40320.0), -1.0 / 720.0), 1.0 / 24.0), -0.5);
+    s = phi * sin_series(x2);
+    cm1 = x2 * cosm1_series(x2);
 }
 // fp32 on |phi| <= 0.03: through phi^3 / phi^4 (truncation < 7e-9 relative,
 // below fp32 rounding)
@@ -180,9 +187,9 @@ __device__ __forceinline__ void sin_cosm1_tiny(double phi, double& s, double& cm
 // library's sincos otherwise
 __device__ __forceinline__ void sincos_turn(double x, double& s, double& c) {
     if (fabs(x) <= 0.0625) {
-        double cm1;
-        sin_cosm1_small(x, s, cm1);
-        c = 1.0 + cm1;
+        const double x2 = x * x;
+        s = x * sin_series(x2);
+        c = fma(x2, cosm1_series(x2), 1.0);
     } else {
         sincos(x, &s, &c);
     }
@@ -192,7 +199,7 @@ __device__ __forceinline__ void sincos_turn(double x, double& s, double& c) {
 // root otherwise
 __device__ __forceinline__ double inv_norm(double n2) {
     const double e = n2 - 1.0;
-    return fabs(e) < 1e-5 ? 1.0 + e * (-0.5 + 0.375 * e) : 1.0 / sqrt(n2);
+    return fabs(e) < 1e-5 ? fma(e, fma(e, 0.375, -0.5), 1.0) : 1.0 / sqrt(n2);
 }
 template <class T> struct SmallAngle;
 template <> struct SmallAngle<float> { static constexpr float value = 0.1f; };
@@ -490,18 +497,45 @@ __device__ inline void jacobi_agm(double u, double m, const AgmLevels& g, double
 __device__ __forceinline__ int sign_of(double x) { return x >= 0.0 ? 1 : -1; }
 __device__ __forceinline__ int stair(double x) { return x > 0.0 ? (int)ceil(x - 0.5) : (int)floor(x + 0.5); }
 
+// The rotations below stand in several kernels that have to give one
+// trajectory bit for bit, so, as in step_rot and step_apply, every fused
+// operation is written out: of a sum of two products the second is rounded
+// and the first fused, unless the other is written.
+__device__ __forceinline__ double sum_of_products(double a, double b, double c, double d) { return fma(a, b, c * d); }
+// |q|^2
+__device__ __forceinline__ double norm2(Q4<double> q) {
+    return fma(q.d, q.d, fma(q.c, q.c, sum_of_products(q.a, q.a, q.b, q.b)));
+}
+// q (x) z0^* (x) z for z0 = (z0.a, z0.b, z0.c, 0): z dot(z0, q) + C(z) C(z0)^T q
+__device__ __forceinline__ Q4<double> turned(Q4<double> q, double z0a, double z0b, double z0c, Q4<double> z) {
+    const double t = fma(q.c, z0c, sum_of_products(q.a, z0a, q.b, z0b));
+    const double x = fma(q.d, z0c, sum_of_products(q.b, z0a, -q.a, z0b));
+    const double y = fma(-q.d, z0b, sum_of_products(q.c, z0a, -q.a, z0c));
+    const double w = fma(q.d, z0a, sum_of_products(q.c, z0b, -q.b, z0c));
+    return {fma(t, z.a, fma(-w, z.d, sum_of_products(x, -z.b, -y, z.c))),
+            fma(t, z.b, fma(-w, z.c, sum_of_products(x, z.a, y, z.d))),
+            fma(t, z.c, fma(w, z.b, sum_of_products(y, z.a, -x, z.d))),
+            fma(t, z.d, fma(w, z.a, sum_of_products(x, z.c, -y, z.b)))};
+}
+
 // free linear rotor (dof 5): body-frame L constant, rotation about L at
 // |w| = |L| / I0 (closed form; replaces the exact solution, which divides by
 // I0 - I1 = 0 for these bodies)
 __device__ inline void linear_rotor_exact(Q4<double>& q, V3<double> L, V3<double> invI, double dt) {
     V3<double> w = hadamard(invI, L);
-    double wn = sqrt(dot(w, w));
+    double wn = sqrt(fma(w.z, w.z, sum_of_products(w.x, w.x, w.y, w.y)));
     if (wn == 0.0) return;
     double sh, ch;
     sincos_turn(0.5 * wn * dt, sh, ch);
-    V3<double> axis = w * (1.0 / wn);
-    q = q * ch + Bmul(q, axis) * sh;
-    q = q * inv_norm(dot(q, q));
+    V3<double> u = w * (1.0 / wn);
+    // q cos + B(q) u sin
+    const Q4<double> p = {fma(-u.z, q.d, sum_of_products(u.x, -q.b, -u.y, q.c)),
+                          fma(u.z, q.c, sum_of_products(u.x, q.a, -u.y, q.d)),
+                          fma(-u.z, q.b, sum_of_products(u.y, q.a, u.x, q.d)),
+                          fma(u.z, q.a, sum_of_products(u.y, q.b, -u.x, q.c))};
+    q = {sum_of_products(p.a, sh, ch, q.a), sum_of_products(p.b, sh, ch, q.b), sum_of_products(p.c, sh, ch, q.c),
+         sum_of_products(p.d, sh, ch, q.d)};
+    q = q * inv_norm(norm2(q));
 }
 
 // exact free-rotor rotation of (q, L) over dt by the reference's closed form
@@ -517,7 +551,7 @@ __device__ inline void exact_rotation_closed(Q4<double>& q, V3<double>& Lb, V3<d
     const double PI = 3.14159265358979323846;
     V3<double> Iw = Lb;
     V3<double> w0 = hadamard(invI, Iw);
-    double Lsq = Iw.y * Iw.y + Iw.z * Iw.z;
+    double Lsq = sum_of_products(Iw.y, Iw.y, Iw.z, Iw.z);
     if (Lsq < eps) {
         // rotation about body axis 1 only (RigidBody.cpp:246-247): q turns by
         // theta = L1 dt / I1 about e1, L by -theta about e1
@@ -525,16 +559,17 @@ __device__ inline void exact_rotation_closed(Q4<double>& q, V3<double>& Lb, V3<d
         double sh, ch, s2, c2;
         sincos(0.5 * theta, &sh, &ch);
         sincos(theta, &s2, &c2);
-        q = q * ch + perm<1>(q) * sh;
-        Lb = {Iw.x, Iw.y * c2 + Iw.z * s2, -Iw.y * s2 + Iw.z * c2};
+        q = {sum_of_products(q.a, ch, -q.b, sh), sum_of_products(q.a, sh, q.b, ch), sum_of_products(q.c, ch, q.d, sh),
+             sum_of_products(q.d, ch, -q.c, sh)};
+        Lb = {Iw.x, sum_of_products(Iw.y, c2, Iw.z, s2), sum_of_products(Iw.z, c2, -Iw.y, s2)};
         return;
     }
-    Lsq += Iw.x * Iw.x;
+    Lsq = fma(Iw.x, Iw.x, Lsq);
     double L = sqrt(Lsq);
-    double twoKr = dot(Iw, w0);
-    Q4<double> z0 = {Iw.z, Iw.y, L - Iw.x, 0.0};
-    double r1 = Lsq - twoKr * I.z;
-    double r3 = twoKr * I.x - Lsq;
+    double twoKr = sum_of_products(Iw.x, w0.x, Iw.y, w0.y) + product(Iw.z, w0.z);
+    const double z0a = Iw.z, z0b = Iw.y, z0c = L - Iw.x;
+    double r1 = fma(-twoKr, I.z, Lsq);
+    double r3 = fma(twoKr, I.x, -Lsq);
     double l1 = r1 * invI.y / (I.y - I.z);
     double l3 = r3 * invI.y / (I.x - I.y);
     const bool low = l1 < l3;
@@ -572,14 +607,17 @@ __device__ inline void exact_rotation_closed(Q4<double>& q, V3<double>& Lb, V3<d
     double deltaF = u - u0 + sign_of(cn) * omega_fn(sn, npar, m) - sign_of(c0) * om0 +
                     (alpha / C) * (atan(C * sn / (low ? dn : cn)) - atan(C * s0 * a.z / w0.z));
     if (jump != 0) deltaF += jump * (2.0 * omega_fn(1.0, npar, m) + (low ? 0.0 : (alpha / C) * PI));
-    Iw = low ? hadamard(Ia, V3<double>{cn, sn, dn}) : hadamard(Ia, V3<double>{dn, sn, cn});
+    const double e1 = low ? cn : dn;
+    Iw = {Ia.x * e1, Ia.y * sn, Ia.z * (low ? dn : cn)};
     deltaF *= 1.0 + eta;
-    double theta = (Lsq * (u - u0) + r3 * deltaF) / (2.0 * L * I.x * wp);
+    double theta = sum_of_products(Lsq, u - u0, r3, deltaF) / (2.0 * L * I.x * wp);
     double st, ct;
     sincos(theta, &st, &ct);
-    Q4<double> z = Q4<double>{Iw.z, Iw.y, L - Iw.x, 0.0} * ct + Q4<double>{-Iw.y, Iw.z, 0.0, L - Iw.x} * st;
-    q = z * dot(z0, q) + Cmul(z, Ctmul(z0, q));
-    double r = 1.0 / sqrt(dot(q, q));
+    // z = (L3, L2, |L| - L1, 0) cos + (-L2, L3, 0, |L| - L1) sin
+    const double z2 = fma(-Ia.x, e1, L);
+    q = turned(q, z0a, z0b, z0c,
+               {sum_of_products(Iw.z, ct, -Iw.y, st), sum_of_products(Iw.y, ct, Iw.z, st), z2 * ct, z2 * st});
+    double r = 1.0 / sqrt(norm2(q));
     q = q * r;
     Lb = Iw;
 }
@@ -696,16 +734,16 @@ __device__ inline void exact_rotation(Q4<double>& q, V3<double>& Lb, V3<double> 
     const bool flip = Lb.x > 0.0;
     V3<double> Iw = flip ? V3<double>{-Lb.x, -Lb.y, Lb.z} : Lb;
     V3<double> w0 = hadamard(invI, Iw);
-    double Lsq = Iw.y * Iw.y + Iw.z * Iw.z;
+    double Lsq = sum_of_products(Iw.y, Iw.y, Iw.z, Iw.z);
     // (L along e1: the closed form too, from one place, since its code and its
     // constants' registers weigh on every kernel that holds a call: 512 waters
     // in FP64, 100 steps, 365 -> 353 us; the 200k-body mix, 250 steps, 5.0 -> 4.7 ms)
     const bool axial = Lsq < eps;
-    Lsq += Iw.x * Iw.x;
+    Lsq = fma(Iw.x, Iw.x, Lsq);
     double L = sqrt(Lsq);
-    double twoKr = dot(Iw, w0);
-    double r1 = Lsq - twoKr * I.z;
-    double r3 = twoKr * I.x - Lsq;
+    double twoKr = fma(Iw.z, w0.z, sum_of_products(Iw.x, w0.x, Iw.y, w0.y));
+    double r1 = fma(-twoKr, I.z, Lsq);
+    double r3 = fma(twoKr, I.x, -Lsq);
     double l1 = r1 * invI.y / (I.y - I.z);
     double l3 = r3 * invI.y / (I.x - I.y);
     const bool low = l1 < l3;
@@ -736,27 +774,22 @@ __device__ inline void exact_rotation(Q4<double>& q, V3<double>& Lb, V3<double> 
     auto body_Ln = [&](double x, double& D) {
         double sx, cx, dx;
         jacobi_series<TERMS>(x, J, sx, cx, dx);
-        D = 1.0 - ms0 * s0 * sx * sx;
-        double sn = s0 * cx * dx + sx * c0d0;
-        double cn = c0 * cx - s0 * sx * d0 * dx;
-        double dn = d0 * dx - ms0 * sx * c0 * cx;
+        D = fma(-(ms0 * s0 * sx), sx, 1.0);
+        double sn = sum_of_products(s0 * cx, dx, sx, c0d0);
+        double cn = sum_of_products(c0, cx, -(s0 * sx * d0), dx);
+        double dn = sum_of_products(d0, dx, -(ms0 * sx * c0), cx);
         return low ? V3<double>{Ia.x * cn, Ia.y * sn, Ia.z * dn} : V3<double>{Ia.x * dn, Ia.y * sn, Ia.z * cn};
-    };
-    auto body_L = [&](double x) {
-        double D;
-        V3<double> Ln = body_Ln(x, D);
-        return Ln * (1.0 / D);
     };
     // 2 dtheta/dt at u0 + x, (|L| + L1) X - L1 / I1: X is the same for Ln as
     // for L, so one reciprocal serves X and L1 = Ln1 / D
     auto rate = [&](double x) {
         double D;
         V3<double> Ln = body_Ln(x, D);
-        double y2 = Ln.y * Ln.y, z2 = Ln.z * Ln.z, s2 = y2 + z2;
+        double y2 = Ln.y * Ln.y, z2 = Ln.z * Ln.z, s2 = fma(Ln.y, Ln.y, z2);
         double p = 1.0 / (D * s2);
-        double X = (y2 * invI.y + z2 * invI.z) * D * p;
-        double L1 = Ln.x * s2 * p;
-        return (L + L1) * X - L1 * invI.x;
+        double X = sum_of_products(y2, invI.y, z2, invI.z) * D * p;
+        double n1 = Ln.x * s2;
+        return sum_of_products(X, fma(n1, p, L), -(n1 * p), invI.x);
     };
     // Gauss-Legendre nodes and weights on [-1, 1]: 5 points, or 3 for fp32 state
     const double h = 0.5 * delta;
@@ -764,22 +797,26 @@ __device__ inline void exact_rotation(Q4<double>& q, V3<double>& Lb, V3<double> 
     if constexpr (FP32_STATE) {
         const double gx1 = 0.7745966692414834;
         const double gw0 = 0.8888888888888888, gw1 = 0.5555555555555556;
-        sum = gw0 * rate(h) + gw1 * (rate(h * (1.0 - gx1)) + rate(h * (1.0 + gx1)));
+        sum = sum_of_products(gw0, rate(h), gw1, rate(h * (1.0 - gx1)) + rate(h * (1.0 + gx1)));
     } else {
         const double gx1 = 0.5384693101056831, gx2 = 0.9061798459386640;
         const double gw0 = 0.5688888888888889, gw1 = 0.4786286704993665, gw2 = 0.2369268850561891;
-        sum = gw0 * rate(h) + gw1 * (rate(h * (1.0 - gx1)) + rate(h * (1.0 + gx1))) +
-              gw2 * (rate(h * (1.0 - gx2)) + rate(h * (1.0 + gx2)));
+        sum = fma(gw2, rate(h * (1.0 - gx2)) + rate(h * (1.0 + gx2)),
+                  sum_of_products(gw0, rate(h), gw1, rate(h * (1.0 - gx1)) + rate(h * (1.0 + gx1))));
     }
     double theta = 0.25 * dt * sum;
-    V3<double> Iw1 = body_L(delta);
-    Q4<double> z0 = {Iw.z, Iw.y, L - Iw.x, 0.0};
+    double D1;
+    const V3<double> Ln = body_Ln(delta, D1);
+    const double rD = 1.0 / D1;
+    V3<double> Iw1 = Ln * rD;
     double st, ct;
     sincos_turn(theta, st, ct);
-    Q4<double> z = Q4<double>{Iw1.z, Iw1.y, L - Iw1.x, 0.0} * ct + Q4<double>{-Iw1.y, Iw1.z, 0.0, L - Iw1.x} * st;
-    Q4<double> qf = flip ? perm<3>(q) : q;
-    qf = z * dot(z0, qf) + Cmul(z, Ctmul(z0, qf));
-    double r = inv_norm(dot(qf, qf));
+    // z = (L3, L2, |L| - L1, 0) cos + (-L2, L3, 0, |L| - L1) sin
+    const double z2 = fma(-rD, Ln.x, L);
+    const Q4<double> z = {sum_of_products(Iw1.z, ct, -Iw1.y, st), sum_of_products(Iw1.z, st, Iw1.y, ct), z2 * ct,
+                          z2 * st};
+    Q4<double> qf = turned(flip ? perm<3>(q) : q, Iw.z, Iw.y, L - Iw.x, z);
+    double r = inv_norm(norm2(qf));
     // P3 P3 q = -q: the turn back is -P3
     q = flip ? perm<3>(qf) * -r : qf * r;
     Lb = flip ? V3<double>{-Iw1.x, -Iw1.y, Iw1.z} : Iw1;

@@ -1601,8 +1601,8 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
 // of once per step.  The arithmetic and every rounding to the state precision
 // are those of k_part1, k_forces and k_fused (the fused operations whose
 // choice the compiler makes by context are written out: step_rot, step_apply,
-// to_body, kicked), so results are the same bit for bit as part 1, then
-// [forces, fused pass], gives.
+// to_body, kicked, the exact rotation), so results are the same bit for bit as
+// part 1, then [forces, fused pass], gives.
 // FIRST: a part 1 comes before the boundaries; LAST: the atom positions are
 // written at the end (a launch that continues another reads only the body
 // state).
