@@ -341,8 +341,10 @@ int rbhip_get_body_fixed_positions(rbhip_context* ctx, double* xyz);
 /* ---------------------------------------------------------------------- */
 /* Launch configuration, autotuning, measurement                           */
 /* ---------------------------------------------------------------------- */
-/* workgroup size (64..1024, multiple of 64) and grid cap (0 = one workgroup
-   per tile) */
+/* workgroup size (64..512, 256 with the exact rotation, multiple of 64) and
+   grid cap (0 = one workgroup per tile) of the step kernels that a call
+   launches one by one; the steps that rbhip_execute keeps in registers always
+   run in one-wave workgroups, one per tile */
 int rbhip_set_launch(rbhip_context* ctx, int blockSize, int maxBlocks);
 /* lanes per body for the bodies of N atoms (power of two, 1..64) */
 int rbhip_set_lanes(rbhip_context* ctx, int atomsPerBody, int lanes);
@@ -356,9 +358,13 @@ int rbhip_set_lanes(rbhip_context* ctx, int atomsPerBody, int lanes);
    every body's coordinates, RigidBodySystem.cpp:94-95.) */
 int rbhip_set_shared_frames(rbhip_context* ctx, int enable);
 /* times candidate (lanes per body, workgroup size) tiles on a scratch copy of
-   the state and keeps the fastest; the context's state is not advanced */
+   the state and keeps the fastest: the workgroup size by the kernels that read
+   it (part 1, forces, part 2 and, with fusion, the fused pass and its forces),
+   the lanes by those and a step of rbhip_execute together; the context's state
+   is not advanced */
 int rbhip_autotune(rbhip_context* ctx, int reps);
-/* describes the chosen tiling as text */
+/* describes the chosen tiling as text; steps=registers: rbhip_execute keeps
+   the interior steps in registers */
 int rbhip_describe(rbhip_context* ctx, char* buf, int len);
 /* advances the state 2*steps+1 steps on the context's stream: `steps`
    two-pass steps (part1, forces, part2), then the fused path of

@@ -358,12 +358,51 @@ void time_phases(hipStream_t stream, int steps, const std::vector<std::function<
     }
 }
 
-// boundaries of a launchSteps call that a tuner times
-constexpr int kTuneBoundaries = 16;
-
 template <class P1, class F, class P2>
 void time_steps(hipStream_t stream, int steps, P1 p1, F f, P2 p2, double* avgMs, double* totalMs) {
     time_phases(stream, steps, {p1, f, p2}, avgMs, totalMs);
+}
+
+// What a tuner compares, in ms per step, for any candidate and whichever path
+// its steps take:
+// - the step kernels one by one, as the calls of a half step, and steps with
+//   bonds or other forces, launch them (part 1, forces, part 2; with `fused`
+//   the fused pass and its forces too);
+template <class O> double time_step_kernels(O& o, int reps, bool fused) {
+    double avg[3], sum;
+    o.launchPart1();
+    o.launchForces();
+    o.launchPart2();
+    time_steps(o.stream, reps, [&] { o.launchPart1(); }, [&] { o.launchForces(false); }, [&] { o.launchPart2(); }, avg,
+               nullptr);
+    sum = avg[0] + avg[1] + avg[2];
+    if (fused) {
+        o.launchPart1();
+        o.launchForces();
+        o.launchFused();
+        o.launchForces();
+        time_phases(o.stream, reps, {[&] { o.launchFused(); }, [&] { o.launchForces(false); }}, avg, nullptr);
+        o.launchPart2();
+        sum += avg[0] + avg[1];
+    }
+    return sum;
+}
+// - a step of a call of kTuneSteps steps, all of its kernels and gaps included
+//   (the fastest of `reps` calls; too short for a graph).
+constexpr int kTuneSteps = 17;
+template <class O> double time_execute(O& o, int reps) {
+    EventSet span(2);
+    double best = 1e300;
+    for (int r = 0; r <= reps; r++) {
+        HIPCHK(hipEventRecord(span.ev[0], o.stream));
+        run_steps(o, kTuneSteps, false);
+        HIPCHK(hipEventRecord(span.ev[1], o.stream));
+        HIPCHK(hipEventSynchronize(span.ev[1]));
+        float ms = 0.f;
+        HIPCHK(hipEventElapsedTime(&ms, span.ev[0], span.ev[1]));
+        if (r > 0) best = std::min(best, (double)ms / kTuneSteps);   // (r = 0: warm-up)
+    }
+    return best;
 }
 }  // namespace
 
@@ -2560,7 +2599,8 @@ int rbhip_describe(rbhip_context* ctx, char* buf, int len) {
             s += "N" + std::to_string(c.N) + "x" + std::to_string(c.count) + ":L" +
                  std::to_string(it == ctx->lanes.end() ? 1 : it->second) + " ";
         }
-        s += "] free=" + std::to_string(ctx->numFree);
+        s += "] free=" + std::to_string(ctx->numFree) +
+             " steps=" + (ctx->useFusion && ctx->localSteps() ? "registers" : "launched");
         std::string shapes;
         for (auto& c : ctx->classes)
             if (c.shapes > 0) shapes += " N" + std::to_string(c.N) + ":" + std::to_string(c.shapes);
@@ -2617,29 +2657,14 @@ int rbhip_autotune(rbhip_context* ctx, int reps) {
             C.restoreSnapshot(snap, C.stream);
             HIPCHK(hipStreamSynchronize(C.stream));
         };
-        // the time of what rbhip_execute launches: a few steps in registers
-        // and their last forces and part 2 where it can, the fused pass +
-        // forces of one step with fusion, part1 + forces + part2 without
-        auto measure = [&]() -> double {
-            double avg[3], total;
-            double t;
-            if (C.useFusion && C.localSteps()) {
-                C.launchSteps(kTuneBoundaries); C.launchForces(); C.launchPart2();
-                time_phases(C.stream, reps, {[&] { C.launchSteps(kTuneBoundaries); }, [&] { C.launchForces(true); },
-                                             [&] { C.launchPart2(); }}, avg, &total);
-                t = avg[0] + avg[1] + avg[2];
-            } else if (C.useFusion) {
-                C.launchPart1(); C.launchForces();
-                C.launchFused(); C.launchForces();
-                time_phases(C.stream, reps, {[&] { C.launchFused(); }, [&] { C.launchForces(false); }}, avg, &total);
-                C.launchPart2();
-                t = avg[0] + avg[1];
-            } else {
-                C.launchPart1(); C.launchForces(); C.launchPart2();
-                time_steps(C.stream, reps, [&] { C.launchPart1(); }, [&] { C.launchForces(false); },
-                           [&] { C.launchPart2(); }, avg, &total);
-                t = avg[0] + avg[1] + avg[2];
-            }
+        // the workgroup size by the kernels that read it (the steps in
+        // registers do not); the lanes, which every path reads, by those and
+        // a step of rbhip_execute (200k mixed bodies, exact rotation, the
+        // 20-atom bodies on 2 lanes instead of 4: k_steps 8.8 -> 7.6 us a
+        // step, but part 2 15.2 -> 17.0 and the fused pass 21.9 -> 23.2)
+        auto measure = [&](bool execute) -> double {
+            double t = time_step_kernels(C, reps, C.useFusion);
+            if (execute) t += time_execute(C, reps);
             restore();
             return t;
         };
@@ -2654,7 +2679,7 @@ int rbhip_autotune(rbhip_context* ctx, int reps) {
                 if (!ok) continue;
                 C.block = b;
                 C.rebuildTiles();
-                double t = measure();
+                double t = measure(false);
                 if (t < best) { best = t; bestBlock = b; }
             }
             C.block = bestBlock;
@@ -2667,7 +2692,7 @@ int rbhip_autotune(rbhip_context* ctx, int reps) {
                     if (C.block % L) continue;
                     C.lanes[cl.N] = L;
                     C.rebuildTiles();
-                    double t = measure();
+                    double t = measure(true);
                     if (t < bestT) { bestT = t; bestL = L; }
                 }
                 C.lanes[cl.N] = bestL;
@@ -2896,26 +2921,21 @@ int rbhip_batch_autotune(rbhip_batch* batch, int reps) {
             for (size_t m = 0; m < B.members.size(); m++) B.members[m]->restoreSnapshot(*snaps[m], B.stream);
             HIPCHK(hipStreamSynchronize(B.stream));
         };
-        // time of what rbhip_batch_execute launches, as in rbhip_autotune
-        auto measure = [&]() -> double {
-            double avg[3], total, t;
+        // as in rbhip_autotune; of a batch's kernels, steps in registers leave
+        // the forces and part 2 at their end
+        auto measure = [&](bool execute) -> double {
+            double t;
             if (B.useFusion && B.localSteps()) {
-                B.launchSteps(kTuneBoundaries); B.launchForces(); B.launchPart2();
-                time_phases(B.stream, reps, {[&] { B.launchSteps(kTuneBoundaries); }, [&] { B.launchForces(true); },
-                                             [&] { B.launchPart2(); }}, avg, &total);
-                t = avg[0] + avg[1] + avg[2];
-            } else if (B.useFusion) {
-                B.launchPart1(); B.launchForces();
-                B.launchFused(); B.launchForces();
-                time_phases(B.stream, reps, {[&] { B.launchFused(); }, [&] { B.launchForces(false); }}, avg, &total);
+                double avg[2];
+                B.launchSteps(1);
+                B.launchForces();
                 B.launchPart2();
+                time_phases(B.stream, reps, {[&] { B.launchForces(true); }, [&] { B.launchPart2(); }}, avg, nullptr);
                 t = avg[0] + avg[1];
             } else {
-                B.launchPart1(); B.launchForces(); B.launchPart2();
-                time_steps(B.stream, reps, [&] { B.launchPart1(); }, [&] { B.launchForces(false); },
-                           [&] { B.launchPart2(); }, avg, &total);
-                t = avg[0] + avg[1] + avg[2];
+                t = time_step_kernels(B, reps, B.useFusion);
             }
+            if (execute) t += time_execute(B, reps);
             restore();
             return t;
         };
@@ -2937,7 +2957,7 @@ int rbhip_batch_autotune(rbhip_batch* batch, int reps) {
                     B.block = blk;
                     B.maxBlocks = grid;
                     B.rebuild();
-                    double t = measure();
+                    double t = measure(false);
                     if (t < best) { best = t; bestBlock = blk; bestGrid = grid; }
                 }
             }
@@ -2960,7 +2980,7 @@ int rbhip_batch_autotune(rbhip_batch* batch, int reps) {
                                                              [&](const rbhip_context::Class& cl) { return cl.N == N; }))
                             c->lanes[N] = L;
                     B.rebuild();
-                    double t = measure();
+                    double t = measure(true);
                     if (t < bestT) { bestT = t; bestL = L; }
                 }
                 for (rbhip_context* c : B.members)
