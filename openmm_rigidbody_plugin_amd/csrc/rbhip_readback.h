@@ -82,8 +82,10 @@ struct PinnedLease {
 // copies `bytes` at device address src to dst after the work queued on
 // `stream`, and waits for it.  Threads: one per 2 chunks, at most 4 (1M
 // waters' positions, 72 MB into fresh memory: 6.9 ms direct, 2.6 with 3
-// threads, 2.1-2.2 with 4, 6, 8 or 12; chunks of 1 MiB: 2.6).  One chunk (512
-// waters' positions: 44 us direct, 29 pinned) needs no other thread.
+// threads, 2.1-2.2 with 4, 6, 8 or 12; chunks of 1 MiB: 2.6).  One chunk needs
+// no other thread (14 KB: 44 us direct, 29 pinned).  The other threads' copies
+// wait for an event that the caller records: a handle such as
+// hipStreamPerThread names another stream in each of them.
 inline hipError_t read_back(void* dst, const void* src, size_t bytes, int device, hipStream_t stream) {
     constexpr size_t chunk = PinnedChunks::kBytes;
     const size_t count = (bytes + chunk - 1) / chunk;
@@ -101,9 +103,19 @@ inline hipError_t read_back(void* dst, const void* src, size_t bytes, int device
     // thread t empties chunks t, t + threads, ... through its two buffers
     const int threads = (int)lease.chunks.size() / 2;
     std::vector<hipError_t> status(threads, hipSuccess);
+    struct Event {
+        hipEvent_t ev = nullptr;
+        ~Event() {
+            if (ev) (void)hipEventDestroy(ev);
+        }
+    } ready;   // what was queued on the caller's stream
+    hipError_t r = hipEventCreateWithFlags(&ready.ev, hipEventDisableTiming);
+    if (r == hipSuccess) r = hipEventRecord(ready.ev, stream);
+    if (r != hipSuccess) return r;
     auto worker = [&](int t) {
         hipError_t& e = status[t];
         e = hipSetDevice(device);
+        if (e == hipSuccess) e = hipStreamWaitEvent(stream, ready.ev, 0);
         hipEvent_t done[2] = {nullptr, nullptr};
         for (int b = 0; b < 2 && e == hipSuccess; b++) e = hipEventCreateWithFlags(&done[b], hipEventDisableTiming);
         auto issue = [&](size_t c, int b) {
