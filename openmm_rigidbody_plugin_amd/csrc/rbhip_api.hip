@@ -524,7 +524,7 @@ struct rbhip_context {
     Tile* dSetupTiles = nullptr;
     Tile* dStepTiles = nullptr;                  // part tiles of kStepsBlock threads, for launchSteps
     int atomsPerLane = 0;                        // the most body atoms a lane holds in them
-    int nPartTiles = 0, nForceTiles = 0, nSetupTiles = 0, nStepTiles = 0;
+    int nPartTiles = 0, nForceTiles = 0, nSetupTiles = 0, nStepTiles = 0, nStepBodyTiles = 0;
     // cluster tiles, 64 clusters each: KE slots after the part tiles, and a
     // copy whose slots follow the set-up tiles
     Tile* dClusterTiles = nullptr;
@@ -691,6 +691,10 @@ struct rbhip_context {
         return m;
     }
 
+    static int bodyTilesOf(const std::vector<Tile>& tiles) {
+        return (int)std::count_if(tiles.begin(), tiles.end(), [](const Tile& t) { return t.kind == TILE_BODIES; });
+    }
+
     std::vector<Tile> forceTiles(int blk) const {
         std::vector<Tile> t;
         const int atomTile = FORCE_PER_THREAD * blk;
@@ -811,6 +815,7 @@ struct rbhip_context {
             HIPCHK(hipMemcpyAsync(table, all.data(), all.size() * sizeof(Tile), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
         atomsPerLane = mostPerLane(block == kStepsBlock ? pt : kt);
+        nStepBodyTiles = bodyTilesOf(block == kStepsBlock ? pt : kt);
         nStepTiles = block == kStepsBlock ? (int)pt.size() : (int)kt.size();
         nPartTiles = (int)pt.size();
         nForceTiles = (int)ft.size();
@@ -878,15 +883,17 @@ struct rbhip_context {
         launchSites();
     }
     // whether launchSteps can carry the system through several steps at once:
-    // no atom's force depends on another atom, and a lane's atoms fit its LDS
-    // (a site belongs to its body, a cluster is a whole of its own)
+    // no atom's force depends on another atom (a site belongs to its body, a
+    // cluster is a whole of its own), a lane's atoms fit its LDS, and that
+    // leaves waves enough
     bool localSteps() const {
         if (h.bondStart || (numSites > 0 && h.maxBodySites == 0) || clusterClassTiles[3] > 0) return false;
         for (int n : siteBodySizes) {
             auto it = lanes.find(n);
             if (it != lanes.end() && it->second > 1) return false;   // (one lane has the body's atoms)
         }
-        return steps_lds_bytes(precision, atomsPerLane, h.maxBodySites) <= kStepsLdsMax;
+        const size_t lds = steps_lds_bytes(precision, atomsPerLane, h.maxBodySites);
+        return lds <= kStepsLdsMax && steps_lds_pays(precision, lds, nStepBodyTiles);
     }
     void launchSteps(int boundaries) {
         if (nClusterTiles > 0)
@@ -1170,7 +1177,7 @@ struct rbhip_batch {
     Tile* dPartTiles = nullptr;
     Tile* dForceTiles = nullptr;
     Tile* dStepTiles = nullptr;                  // as a context's, over the members
-    int nPart = 0, nForce = 0, nStep = 0;
+    int nPart = 0, nForce = 0, nStep = 0, nStepBody = 0;
     int atomsPerLane = 0;                        // of the step tiles, as built
     std::vector<int> memberPartTiles, memberForceTiles;
     std::vector<int> memberVersions;             // sysVersion of each member's DevSys copy
@@ -1181,7 +1188,8 @@ struct rbhip_batch {
 
     void rebuild() {
         arena.release();
-        nPart = nForce = nStep = 0;
+        nPart = nForce = nStep = nStepBody = 0;
+        atomsPerLane = 0;
         memberPartTiles.assign(members.size(), 0);
         memberForceTiles.assign(members.size(), 0);
         if (members.empty()) return;
@@ -1228,6 +1236,7 @@ struct rbhip_batch {
         HIPCHK(hipStreamSynchronize(stream));
         nStep = block == kStepsBlock ? (int)pt.size() : (int)kt.size();
         atomsPerLane = rbhip_context::mostPerLane(block == kStepsBlock ? pt : kt);
+        nStepBody = rbhip_context::bodyTilesOf(block == kStepsBlock ? pt : kt);
         nPart = (int)pt.size();
         nForce = (int)ft.size();
     }
@@ -1264,7 +1273,8 @@ struct rbhip_batch {
     bool localSteps() const {
         for (const rbhip_context* c : members)
             if (c->h.bondStart || c->numSites > 0 || c->numClusters > 0) return false;
-        return steps_lds_bytes(precision, atomsPerLane, 0) <= kStepsLdsMax;
+        const size_t lds = steps_lds_bytes(precision, atomsPerLane, 0);
+        return lds <= kStepsLdsMax && steps_lds_pays(precision, lds, nStepBody);
     }
     void launchSteps(int boundaries) {
         HIPCHK(launch_steps(precision, rotationMode, dSystems, dStepTiles, nStep, boundaries, atomsPerLane, 0, stream,

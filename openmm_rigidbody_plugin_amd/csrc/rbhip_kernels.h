@@ -45,6 +45,9 @@ constexpr size_t kStepsLdsMax = 64 << 10;
 constexpr int kSiteReals = 14;        // LDS of a site, in state-precision values
 constexpr int kMaxSiteBody = 1000;    // atoms of a body with such sites
 size_t steps_lds_bytes(int precision, int atomsPerLane, int sitesPerLane);
+// whether that LDS leaves the workgroups of bodyTiles tiles of bodies enough
+// waves per CU for the steps in registers to be the faster way
+bool steps_lds_pays(int precision, size_t lds, int bodyTiles);
 hipError_t launch_steps(int precision, int rotationMode, const DevSys* systems, const Tile* tiles, int numTiles,
                         int boundaries, int atomsPerLane, int sitesPerLane, hipStream_t stream, int adopted);
 // the same with the system's constraint clusters (tiles and counts as for

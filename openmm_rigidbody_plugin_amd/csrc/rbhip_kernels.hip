@@ -2263,6 +2263,24 @@ size_t steps_lds_bytes(int precision, int atomsPerLane, int sitesPerLane) {
     return (size_t)kStepsBlock * (reals | 1) * (precision == 0 ? sizeof(float) : sizeof(double));
 }
 
+// One-wave workgroups that a CU's LDS holds, of `lds` bytes each.
+static int waves_by_lds(size_t lds) { return (int)((size_t(160) << 10) / lds); }
+
+// Every workgroup of a launch reserves the LDS of its largest bodies' lanes, so
+// one body of hundreds of atoms (16 lanes at most by default) takes the other
+// bodies' waves.  Steps in registers and launched, us a step, beside a body of
+// 280, 400 and 500 atoms in mixed precision (4, 3 and 2 waves per CU): 1M waters
+// under NO-SQUISH(10) 46, 59 and 85, launched 59 to 60; exact rotation 44, 54
+// and 73, launched 70; 300k waters 16, 20 and 28, launched 25 to 26; 100k waters
+// 7, 9 and 11.5, launched 18 to 21; 200k mixed bodies (4063 tiles) 16, 19 and 27,
+// launched 33.  So at 2 waves at most 8 turns.  In double precision, where a
+// launched step moves twice the bytes, the registers win at 2 waves too (1M
+// waters and 280 atoms 104 and 92, launched 136 and 131).
+bool steps_lds_pays(int precision, size_t lds, int bodyTiles) {
+    const int waves = waves_by_lds(lds);
+    return precision != 0 || waves >= 3 || bodyTiles <= 8 * 256 * waves;
+}
+
 // (boundaries, flags) of the launches that carry a system through
 // `boundaries` step boundaries, the last one's with STEPS_LAST
 template <class Launch> static hipError_t steps_launches(int boundaries, Launch&& launch) {
@@ -2309,10 +2327,12 @@ static void cluster_steps_classes(const DevSys* systems, const Tile* tiles, cons
 // One launch for both takes as long as the longer, where two take the sum
 // (10k four-site waters and 2000 triangles, 49 boundaries: 203 + 342 us, 345
 // together).  Its registers allow 2 waves per SIMD, where the bodies alone run
-// 4: so while all of its workgroups are resident at once on 1024 SIMDs.
-// Clusters of 4 atoms need more registers than that.
-static bool steps_together(int numTiles, const int* counts) {
-    return counts[2] == 0 && numTiles + counts[0] + counts[1] <= 2048;
+// 4, and every workgroup has the bodies' LDS: so while all of its workgroups
+// are resident at once on 256 CUs.  Clusters of 4 atoms need more registers
+// than that.
+static bool steps_together(int numTiles, const int* counts, size_t lds) {
+    const int waves = waves_by_lds(lds);
+    return counts[2] == 0 && numTiles + counts[0] + counts[1] <= 256 * (waves < 8 ? waves : 8);
 }
 
 hipError_t launch_steps_with_clusters(int precision, int rotationMode, const DevSys* systems, const Tile* tiles,
@@ -2320,7 +2340,7 @@ hipError_t launch_steps_with_clusters(int precision, int rotationMode, const Dev
                                       int atomsPerLane, int sitesPerLane, hipStream_t stream) {
     const size_t lds = steps_lds_bytes(precision, atomsPerLane, sitesPerLane);
     if (lds > kStepsLdsMax || counts[3]) return hipErrorInvalidValue;
-    if (steps_together(numTiles, counts)) {
+    if (steps_together(numTiles, counts, lds)) {
         const int nc = counts[0] + counts[1];
         return steps_launches(boundaries, [&](int n, int flags) {
             auto go = [&](auto kernel) {
