@@ -12,9 +12,11 @@ step, up to 64 of them per launch.  The step kernels that run one step at a
 time (part1, forces, part2, fused) are timed beside it.
 
 Prints one JSON line: whole-job body-steps/s over K timed steps (inputs
-resident in HBM), the HBM roofline of the dominant integrator kernel measured
-with HIP events on its stream, and the FP64 CPU restatement timed on a bounded
-sample of the same workload on this host.
+resident in HBM), the roofline of the timed region's kernel (steps in
+registers: VALU issue and HBM traffic, from recorded counters and the measured
+time per step), the HBM roofline of the fused pass measured with HIP events on
+its stream, and the FP64 CPU restatement timed on a bounded sample of the same
+workload on this host.
 """
 from __future__ import annotations
 
@@ -32,6 +34,10 @@ sys.path.insert(0, ROOT)
 
 
 HBM_PEAK_GBS = 8000.0   # MI355X published HBM3E bandwidth
+# wave64 VALU instructions that MI355X issued at the most, in 1e9/s: independent
+# fp32 FMAs on vector registers, 64 waves per CU, 1.82 per CU and clock of 2.4 GHz
+# (0.97 with an operand from a scalar register, 0.86 for FP64 FMAs with one)
+VALU_PEAK_G = 1120.0
 
 
 def log(*a):
@@ -189,25 +195,39 @@ def cpu_baseline(spec, budget_s=15.0, sample_bodies=100_000):
                                      **small}}
 
 
-def valu_from_profiles(config, kernel):
-    """VALU issue fraction recorded in profiles/ (rocprofv3 counters of an
-    earlier run of this kernel; not measured by this run)."""
-    path = os.path.join(ROOT, "profiles", f"valu_{kernel}_{config}.json")
+def recorded(what, kernel, config):
+    """A rocprofv3 record under profiles/ (`what`: valu or traffic) of an
+    earlier run of this kernel on this workload, not measured by this run; {}
+    without one."""
+    path = os.path.join(ROOT, "profiles", f"{what}_{kernel}_{config}.json")
     if not os.path.exists(path):
-        return None
+        return {}
     with open(path) as f:
-        return json.load(f).get("valu_issue_frac")
+        return json.load(f)
 
 
-def traffic_from_profiles(config, kernel):
-    """HBM bytes per launch recorded in profiles/ (two rocprofv3 --pmc runs,
-    FETCH_SIZE and WRITE_SIZE scaled by a copy kernel's; not measured by this
-    run)."""
-    path = os.path.join(ROOT, "profiles", f"traffic_{kernel}_{config}.json")
-    if not os.path.exists(path):
-        return None
-    with open(path) as f:
-        return json.load(f).get("bytes_per_launch")
+def steps_roofline(ms_per_step, natoms_body, nb, nf, config, bound="valu issue"):
+    """The timed region's kernel: up to 64 [forces, part2 + part1] per launch
+    with the body state in registers, so a step's bytes are a 64th of a
+    launch's.  Time per step from the timed region (its last forces and part 2
+    included), instructions and traffic from the recorded counters of a launch
+    of 64.  Beside it the bytes that the canonical step (fused pass and forces)
+    would move, over the same time."""
+    valu, traffic = recorded("valu", "steps", config), recorded("traffic", "steps", config)
+    s = ms_per_step * 1e-3
+    canonical = algorithmic_bytes("fused", natoms_body, nb, nf) + algorithmic_bytes("forces", natoms_body, nb, nf)
+    out = {"bound": bound, "kernel": "steps", "boundaries_per_launch": 64, "ms_per_step": ms_per_step,
+           "achieved": None, "peak": VALU_PEAK_G, "unit": "G wave64 VALU instructions/s", "frac": None,
+           "traffic": traffic.get("bytes_per_launch"), "frac_hbm": None,
+           "recorded": f"profiles/kernels_{config}.md (rocprofv3 --pmc, not this run)" if valu and traffic else None,
+           "canonical_bytes_per_step": canonical, "canonical_GBs": canonical / s / 1e9,
+           "canonical_frac_hbm": canonical / s / 1e9 / HBM_PEAK_GBS}
+    if valu:
+        out["achieved"] = valu["valu_instr_per_launch"] / valu["boundaries_per_launch"] / s / 1e9
+        out["frac"] = out["achieved"] / VALU_PEAK_G
+    if traffic:
+        out["frac_hbm"] = traffic["bytes_per_launch"] / traffic["boundaries_per_launch"] / s / 1e9 / HBM_PEAK_GBS
+    return out
 
 
 def plain_run(ctxs, steps, per_step):
@@ -426,11 +446,11 @@ def served_fp64_check(check, bodies=64, free=64, tol_nm=1e-5):
 
 
 def kernel_roofline(kms, natoms_body, nb, nf, config, shared_frames=False):
-    """The HBM roofline of the dominant kernel of step(K) (the fused pass)
-    from its duration (HIP events on its own dispatch) and its algorithmic
-    bytes; the two-pass step
-    (part1 + part2, what one execute() with forces computed outside the
-    library runs) and the full step with the tether beside it."""
+    """The HBM roofline of the fused pass (the interior steps of systems with
+    bonds; these workloads' own steps run in registers, steps_roofline) from
+    its duration (HIP events on its own dispatch) and its algorithmic bytes;
+    the two-pass step (part1 + part2, what one execute() with forces computed
+    outside the library runs) and the full step with the tether beside it."""
     alg = {k: algorithmic_bytes(k, natoms_body, nb, nf) for k in ("part1", "part2", "fused", "forces")}
     impl = {k: implementation_bytes(k, natoms_body, nb, nf, shared_frames) for k in ("part1", "part2", "fused", "forces")}
     achieved = {k: alg[k] / (kms[k] * 1e-3) / 1e9 for k in alg}
@@ -438,21 +458,21 @@ def kernel_roofline(kms, natoms_body, nb, nf, config, shared_frames=False):
     two_ms = kms["part1"] + kms["part2"]
     two_alg = alg["part1"] + alg["part2"]
     return {
-        "roofline": {
+        "roofline_fused": {
             "bound": "hbm",
             "kernel": dominant,
             "achieved": achieved[dominant],
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": achieved[dominant] / HBM_PEAK_GBS,
-            "traffic": traffic_from_profiles(config, dominant),
+            "traffic": recorded("traffic", dominant, config).get("bytes_per_launch"),
             "traffic_source": "recorded: profiles/traffic_fused_" + config + ".json (rocprofv3 --pmc, not this run)",
             "algorithmic_bytes_per_launch": alg[dominant],
             "implementation_bytes_per_launch": impl[dominant],
             "implementation_over_algorithmic": impl[dominant] / alg[dominant],
             "shared_frames": shared_frames,
             "avg_launch_ms": kms[dominant],
-            "valu_issue_frac_recorded": valu_from_profiles(config, dominant),
+            "valu_issue_frac_recorded": recorded("valu", dominant, config).get("valu_issue_frac"),
         },
         "integrator": {
             "note": "the kernels that take one step at a time: the fused pass (interior steps of systems with "
@@ -549,11 +569,13 @@ def hetero_leg(steps, warmup):
     ke = ctx.kinetic_energies()
     assert np.all(np.isfinite(ke)), "non-finite kinetic energy"
     log(f"  hetero200k: {el / steps * 1e3:.4f} ms/step, fused {kms['fused']:.4f} ms, "
-        f"frac {roof['roofline']['frac']:.3f}")
+        f"frac {roof['roofline_fused']['frac']:.3f}")
     return {"workload": cfg["workload"], "bodies": nb, "free_atoms": nf, "steps": steps,
             "ms_per_step": el / steps * 1e3, "value": nb * steps / el, "unit": "body-steps/s",
             "free_atom_steps_per_s": nf * steps / el, "launch": ctx.describe(), "kernel_ms": kms,
-            "roofline": roof["roofline"], "integrator": roof["integrator"]}
+            "roofline": steps_roofline(el / steps * 1e3, counts["numBodyAtoms"] / max(nb, 1), nb, nf, "hetero200k",
+                                       bound="valu latency (the exact rotation's FP64 chains)"),
+            "roofline_fused": roof["roofline_fused"], "integrator": roof["integrator"]}
 
 
 def main():
@@ -648,7 +670,8 @@ def main():
         "dtype": "f32 state, f64 accumulation (mixed)",
         "data": "synthetic (seeded lattice, Maxwell-Boltzmann 300 K, harmonic tethers)",
         "config": {**cfg, "parallelism": "single GPU", "launch": ctx.describe()},
-        "roofline": roof["roofline"],
+        "roofline": steps_roofline(ms_per_step, natoms_body, nb, nf, args.config),
+        "roofline_fused": roof["roofline_fused"],
         "kernel_ms": kms,
         "integrator": roof["integrator"],
     }
