@@ -284,14 +284,29 @@ int rbhip_part2(rbhip_context* ctx);
 /* RigidBodyIntegrator::step(steps) (RigidBodyIntegrator.cpp:96-101).
    With fusion (default) the interior step boundaries run as one pass each:
    part1, forces, (steps-1) x [fused part2+part1, forces], part2 -- the same
-   trajectory as steps x [part1, forces, part2] (bit for bit in mixed
-   precision, to a few ulp in FP64), without the interior steps' atom
-   velocities and kinetic energies, which nothing reads.
-   Without bonds, and with every virtual site a two- or three-particle average
-   of one body's atoms and every cluster of constraints of at most 4 atoms,
-   the interior boundaries run up to 64 per launch with the state in
-   registers.  Long sequences of steps with other sites or clusters are
-   replayed from a HIP graph when enabled. */
+   trajectory as steps x [part1, forces, part2], without the interior steps'
+   atom velocities and kinetic energies, which nothing reads.  In FP64 the two
+   agree to a few ulp.  In mixed precision they agree bit for bit but for rare
+   differences of one fp32 unit: bodies of 2 and 3 atoms under NO-SQUISH, whose
+   positions part 1 and the fused pass round apart in FP64, one body in ~3e7
+   per step; other bodies less than one in 1e9; in adopted arrays also the last
+   bits of posqCorrection.
+
+   The interior boundaries run up to 64 per launch with the state in registers
+   (rbhip_describe: steps=registers) if
+   - there are no bonds;
+   - every virtual site is a two- or three-particle average of one body's
+     atoms, and one lane holds that body (rbhip_set_lanes; by default bodies
+     of 8 atoms and more take several lanes);
+   - every cluster of constraints has at most 4 atoms;
+   - a lane's atoms fit its share of LDS: 36 body atoms per lane in mixed
+     precision and 18 in double, fewer with sites;
+   - in mixed precision, that LDS leaves a CU at least 3 waves, or the body
+     tiles are few enough to be resident all the same (large systems with a
+     body of more than 30 atoms per lane are launched step by step).
+   Other steps are launched kernel by kernel (steps=launched); with sites or
+   clusters long sequences of them are replayed from a HIP graph when
+   enabled. */
 int rbhip_execute(rbhip_context* ctx, int steps);
 /* 1 = capture the repeated launches of long sequences in a HIP graph and
    replay it where that is faster (default) */

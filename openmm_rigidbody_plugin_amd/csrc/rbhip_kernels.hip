@@ -1610,12 +1610,12 @@ __global__ __launch_bounds__(512) void k_forces(const DevSys* __restrict__ syste
 // What bounds it: VALU issue (NO-SQUISH: 41 turns of 24 instructions in the
 // ~1300 of a body's step; FP64 latency with the exact rotation), no longer
 // HBM.  Per step, k_fused + k_forces -> k_steps: 1M waters, NO-SQUISH 10,
-// 58.2 -> 23.4 us; 20k waters 9.9 -> 2.8 us; the heterogeneous mix (200k
-// bodies, 500k free atoms, exact) 32.5 -> 8.6 us; 512 waters in FP64, exact,
-// 9.3 -> 3.2 us.  One wave per workgroup: tiles end apart, and the launch
+// 58.2 -> 24.1 us; 20k waters 9.9 -> 2.8 us; the heterogeneous mix (200k
+// bodies, 500k free atoms, exact) 32.5 -> 8.3 us; 512 waters in FP64, exact,
+// 9.3 -> 2.9 us.  One wave per workgroup: tiles end apart, and the launch
 // fills the SIMDs evenly.  kStepsPerLaunch: 16, 64, 256 and 2048 boundaries
-// per launch ran the 1M waters at 24.0, 23.4, 23.8 and 23.8 us and the
-// heterogeneous mix at 9.2, 8.6, 8.6 and 8.7; 64 leaves other streams a slot
+// per launch ran the 1M waters at 25.7, 24.1, 24.6 and 25.1 us and the
+// heterogeneous mix at 9.0, 8.3, 8.2 and 8.3; 64 leaves other streams a slot
 // every few ms (a server's set-ups: 29 against 31 ms for a backlog with 2048).
 //
 // Sites and clusters (10k four-site waters and 2000 triangles, per step): six

@@ -83,8 +83,8 @@ struct PinnedLease {
 // `stream`, and waits for it.  Threads: one per 2 chunks, at most 4 (1M
 // waters' positions, 72 MB into fresh memory: 6.9 ms direct, 2.6 with 3
 // threads, 2.1-2.2 with 4, 6, 8 or 12; chunks of 1 MiB: 2.6).  One chunk needs
-// no other thread (14 KB: 44 us direct, 29 pinned).  The other threads' copies
-// wait for an event that the caller records: a handle such as
+// no other thread (0.3 to 2 MB: 22 to 115 us, as a direct copy's).  The other
+// threads' copies wait for an event that the caller records: a handle such as
 // hipStreamPerThread names another stream in each of them.
 inline hipError_t read_back(void* dst, const void* src, size_t bytes, int device, hipStream_t stream) {
     constexpr size_t chunk = PinnedChunks::kBytes;
